@@ -74,6 +74,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "oxr_mlp_block_supported": (ctypes.c_int, [_I64, _I64, _I64, _I32]),
     "oxr_mlp_block": (ctypes.c_int, [_P, _I32, _P, _I64, _I64, _I64, _P, _F32, _P, _P, _P, _P, _P, _SZ, _P]),
     "oxr_gemm_bf16": (ctypes.c_int, [_P, _I64, _I64, _P, _I64, _I64, _I32, _P, _I64, _P]),
+    "oxr_gemm_bf16_tall": (ctypes.c_int, [_P, _I64, _I64, _P, _I64, _I64, _I32, _P, _I64, _I32, _P]),
     "oxr_gemm_bf16_partial_splits": (ctypes.c_int32, [_I64, _I64]),
     "oxr_gemm_bf16_partial": (ctypes.c_int, [_P, _I64, _I64, _P, _I64, _I64, _P, _I32, _P]),
     "oxr_lm_head_workspace_bytes": (ctypes.c_size_t, [_I64, _I64]),

@@ -42,8 +42,10 @@
 //                   no workgroup ever waits for another.
 // C layout: lane (l % 16, g) holds rows 4g..4g+3 of the tile for token l % 16.
 #include <algorithm>
+#include <cstdint>
 
 #include "common.h"
+#include "gemm_tile.h"
 #include "lm_head_keys.h"
 
 namespace oxr {
@@ -937,15 +939,18 @@ LaunchConfig choose_config(int64_t n_rows, int64_t K, bool allow_k_splits) {
   return c;
 }
 
-// Token rows one launch of gemm_kernel takes (4 tiles of 16); the entry points take up to kMaxRows
-// and run one launch per 64 rows over the same weight.  The first launch streams the weight from
-// HBM; it is at most a few tens of MB, so the later ones find it in the 256 MB Infinity Cache.
+// Token rows one launch of gemm_kernel takes (4 tiles of 16).  More rows go to the tiled kernel
+// (csrc/gemm_tile.hip): a pass per 64 rows over the weight, as this kernel needs, took at 256 rows 68 us for
+// gate_up (tiled 23), 37 for down_proj (12), 35 for qkv (10) and 18 for o_proj (7.5); at 33 to 64 rows the two
+// are even.  Up to kMaxRows rows the tiled kernel adds the same partial sums in the same order, so a row's
+// result does not depend on how many rows share its call; the packed and the k-split forms take no more.
 constexpr int64_t kPassRows = 64;
 constexpr int64_t kMaxRows = 256;
 
-int check_common(const void* x, int64_t ldx, int64_t M, const void* w, int64_t K, int64_t N) {
+int check_common(const void* x, int64_t ldx, int64_t M, const void* w, int64_t K, int64_t N,
+                 int64_t max_rows = kMaxRows) {
   OXR_RETURN_IF(M < 0 || K <= 0 || N <= 0 || ldx < K, OXR_ERR_INVALID_ARG);
-  OXR_RETURN_IF(M > kMaxRows || K % kKStep != 0, OXR_ERR_UNSUPPORTED);
+  OXR_RETURN_IF(M > max_rows || K % kKStep != 0, OXR_ERR_UNSUPPORTED);
   OXR_RETURN_IF(M > 0 && (!x || !w), OXR_ERR_INVALID_ARG);
   OXR_RETURN_IF(((uintptr_t)x | (uintptr_t)w) % 16 != 0 || ldx % 8 != 0, OXR_ERR_UNSUPPORTED);
   return OXR_OK;
@@ -972,12 +977,12 @@ __global__ __launch_bounds__(256) void pack_weight_kernel(const bf16_t* __restri
 // with row length n; ldy unused; kStore / kSiluMul).  Row-major weights take
 // neither.
 int gemm_entry(const oxr_bf16* x, int64_t ldx, int64_t m, const oxr_bf16* w, int64_t k, int64_t n, int32_t epilogue,
-               oxr_bf16* y, int64_t ldy, bool packed, int32_t flags, oxr_stream_t stream) {
+               oxr_bf16* y, int64_t ldy, bool packed, int32_t flags, int64_t max_rows, oxr_stream_t stream) {
   const bool xp = flags & OXR_GEMM_X_PACKED, yp = flags & OXR_GEMM_Y_PACKED;
   OXR_RETURN_IF((flags & ~(OXR_GEMM_X_PACKED | OXR_GEMM_Y_PACKED)) != 0 || (!packed && flags != 0), OXR_ERR_INVALID_ARG);
   if (xp) ldx = k;
   if (yp) ldy = n;
-  int st = check_common(x, ldx, m, w, k, n);
+  int st = check_common(x, ldx, m, w, k, n, max_rows);
   if (st) return st;
   OXR_RETURN_IF(epilogue != kStore && epilogue != kSiluMul && epilogue != kAddResidual, OXR_ERR_INVALID_ARG);
   OXR_RETURN_IF(!y || ldy < n || ldy % 4 != 0 || (uintptr_t)y % 8 != 0, OXR_ERR_INVALID_ARG);
@@ -987,6 +992,8 @@ int gemm_entry(const oxr_bf16* x, int64_t ldx, int64_t m, const oxr_bf16* w, int
   hipStream_t s = (hipStream_t)stream;
   const LaunchConfig c = choose_config(n, k, false);
   const Layout layout = !packed ? kRowMajor : (xp ? kPackedWX : kPackedW);
+  const TileArgs t{x, ldx, m, w, k, n, y, ldy, nullptr, 1, xp, packed, yp};
+  if (m > kPassRows && gemm_tile_supported(t)) return launch_gemm_tile(t, epilogue, c.waves, m > kMaxRows, s);
   for (int64_t r0 = 0; r0 < m; r0 += kPassRows) {
     // Rows [r0, r0 + 64): a packed operand's rows start r0 * row_length elements in (r0 is a
     // multiple of 16, a whole number of tiles).
@@ -1011,6 +1018,9 @@ int gemm_partial_entry(const oxr_bf16* x, int64_t ldx, int64_t m, const oxr_bf16
   const LaunchConfig c = choose_config(n, k, true);
   OXR_RETURN_IF(k_splits != c.k_splits, OXR_ERR_INVALID_ARG);
   if (m == 0) return OXR_OK;
+  const TileArgs t{x, ldx, m, w, k, n, nullptr, 0, partials, k_splits, xp, packed, false};
+  if (m > kPassRows && gemm_tile_supported(t))
+    return launch_gemm_tile(t, kPartial, c.waves, false, (hipStream_t)stream);
   for (int64_t r0 = 0; r0 < m; r0 += kPassRows) {
     GemmArgs a{x + (xp ? r0 * k : r0 * ldx), ldx, (int)std::min(kPassRows, m - r0), w, k, n, nullptr, 0, 0, nullptr,
                partials + r0 * n, m};
@@ -1119,13 +1129,18 @@ extern "C" int oxr_pack_weight_bf16(const oxr_bf16* w, int64_t rows, int64_t k, 
 
 extern "C" int oxr_gemm_bf16(const oxr_bf16* x, int64_t ldx, int64_t m, const oxr_bf16* w, int64_t k, int64_t n,
                              int32_t epilogue, oxr_bf16* y, int64_t ldy, oxr_stream_t stream) {
-  return oxr::gemm_entry(x, ldx, m, w, k, n, epilogue, y, ldy, false, 0, stream);
+  return oxr::gemm_entry(x, ldx, m, w, k, n, epilogue, y, ldy, false, 0, oxr::kMaxRows, stream);
 }
 
 extern "C" int oxr_gemm_bf16_packed(const oxr_bf16* x, int64_t ldx, int64_t m, const oxr_bf16* w_packed, int64_t k,
                                     int64_t n, int32_t epilogue, oxr_bf16* y, int64_t ldy, int32_t flags,
                                     oxr_stream_t stream) {
-  return oxr::gemm_entry(x, ldx, m, w_packed, k, n, epilogue, y, ldy, true, flags, stream);
+  return oxr::gemm_entry(x, ldx, m, w_packed, k, n, epilogue, y, ldy, true, flags, oxr::kMaxRows, stream);
+}
+
+extern "C" int oxr_gemm_bf16_tall(const oxr_bf16* x, int64_t ldx, int64_t m, const oxr_bf16* w, int64_t k, int64_t n,
+                                  int32_t epilogue, oxr_bf16* y, int64_t ldy, int32_t w_packed, oxr_stream_t stream) {
+  return oxr::gemm_entry(x, ldx, m, w, k, n, epilogue, y, ldy, w_packed != 0, 0, INT64_MAX, stream);
 }
 
 extern "C" int32_t oxr_gemm_bf16_partial_splits(int64_t n, int64_t k) {

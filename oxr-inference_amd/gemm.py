@@ -90,7 +90,7 @@ def pack_weight(w: torch.Tensor) -> PackedMatrix:
 
 EPI_STORE, EPI_SILU_MUL, EPI_ADD_RESIDUAL = 0, 1, 3
 X_PACKED, Y_PACKED = 1, 2  # OXR_GEMM_X_PACKED, OXR_GEMM_Y_PACKED
-MAX_ROWS = 256  # token rows per call (the kernels take 64 per launch over the same weight); more are sliced
+MAX_ROWS = 256  # token rows of a call with packed rows or k-split partials
 
 
 def _tensor(a: Weight) -> torch.Tensor:
@@ -111,24 +111,21 @@ def _check(x: Rows, w: Weight, name: str) -> torch.device:
 
 def _run(x: Rows, w: Weight, n: int, epilogue: int, y: Rows, device: torch.device) -> None:
     m = x.shape[0]
-    if isinstance(w, PackedMatrix):
-        flags = (X_PACKED if isinstance(x, PackedMatrix) else 0) | (Y_PACKED if isinstance(y, PackedMatrix) else 0)
-        if flags:
-            _lib.require(m <= MAX_ROWS, f"packed rows: at most {MAX_ROWS} per call")
-        ldx = 0 if isinstance(x, PackedMatrix) else x.stride(0)
-        ldy = 0 if isinstance(y, PackedMatrix) else y.stride(0)
-        for start in range(0, m, MAX_ROWS):
-            rows = min(MAX_ROWS, m - start)
-            xp = x.data.data_ptr() if isinstance(x, PackedMatrix) else x[start:].data_ptr()
-            yp = y.data.data_ptr() if isinstance(y, PackedMatrix) else y[start:].data_ptr()
-            _lib.call("oxr_gemm_bf16_packed", xp, ldx, rows, w.data.data_ptr(), w.shape[1], n, epilogue, yp, ldy,
-                      flags, _lib.stream(device))
+    if m == 0:
         return
-    _lib.require(not isinstance(y, PackedMatrix), "packed output needs a packed w")
-    for start in range(0, m, MAX_ROWS):
-        rows = min(MAX_ROWS, m - start)
-        _lib.call("oxr_gemm_bf16", x[start:].data_ptr(), x.stride(0), rows, w.data_ptr(), w.shape[1], n, epilogue,
-                  y[start:].data_ptr(), y.stride(0), _lib.stream(device))
+    packed = isinstance(w, PackedMatrix)
+    _lib.require(packed or not isinstance(y, PackedMatrix), "packed output needs a packed w")
+    flags = (X_PACKED if isinstance(x, PackedMatrix) else 0) | (Y_PACKED if isinstance(y, PackedMatrix) else 0)
+    _lib.require(not flags or m <= MAX_ROWS, f"packed rows: at most {MAX_ROWS} per call")
+    ldx = 0 if isinstance(x, PackedMatrix) else x.stride(0)
+    ldy = 0 if isinstance(y, PackedMatrix) else y.stride(0)
+    args = (_tensor(x).data_ptr(), ldx, m, _tensor(w).data_ptr(), w.shape[1], n, epilogue, _tensor(y).data_ptr(), ldy)
+    if m > MAX_ROWS:
+        _lib.call("oxr_gemm_bf16_tall", *args, 1 if packed else 0, _lib.stream(device))
+    elif packed:
+        _lib.call("oxr_gemm_bf16_packed", *args, flags, _lib.stream(device))
+    else:
+        _lib.call("oxr_gemm_bf16", *args, _lib.stream(device))
 
 
 def _check_out(out: Rows, m: int, n: int, name: str) -> None:
