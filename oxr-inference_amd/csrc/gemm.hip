@@ -44,9 +44,11 @@
 #include <algorithm>
 #include <cstdint>
 
+#include "argmax_key.h"
 #include "common.h"
 #include "gemm_tile.h"
 #include "lm_head_keys.h"
+#include "lm_head_wide.h"
 
 namespace oxr {
 namespace {
@@ -54,19 +56,6 @@ namespace {
 enum Epilogue { kStore = 0, kSiluMul = 1, kArgmax = 2, kAddResidual = 3, kPartial = 4 };
 
 constexpr int kKStep = 128;  // k per pipeline stage: 4 MFMA k-steps of 32
-
-// Order-preserving key of a bf16 logit (as fp32 bits) and its column: larger
-// value wins, then lower column.  NaN sorts above everything (torch argmax
-// returns the first NaN); -0 and +0 compare equal.
-__device__ __forceinline__ uint64_t argmax_key(uint32_t fbits, uint32_t col) {
-  uint32_t key;
-  if ((fbits & 0x7fffffffu) > 0x7f800000u) key = 0xffffffffu;
-  else {
-    if ((fbits & 0x7fffffffu) == 0u) fbits = 0u;
-    key = (fbits & 0x80000000u) ? ~fbits : (fbits | 0x80000000u);
-  }
-  return ((uint64_t)key << 32) | (uint32_t)(~col);
-}
 
 __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int mask) {
   const uint32_t lo = __shfl_xor((uint32_t)v, mask, kWave);
@@ -529,261 +518,6 @@ __global__ __launch_bounds__(64 * kLmWaves) void lm_head_lds_kernel(const bf16_t
   }
 }
 
-// ---------------------------------------------------------------------------
-// LM head for 33..256 token rows (packed weight): with M = 256 the head does
-// 159 GFLOP on 622 MB, close to the MFMA/HBM ridge, so the products use the
-// 32x32x16 MFMA (twice the work per issue of the 16x16x32 form on gfx950) and
-// the weight is still read exactly once.  One persistent workgroup per CU
-// owns a balanced contiguous range of 32-row vocab tiles, taken 8 at a time
-// (a group): wave w multiplies vocab tile w of the group by all token rows
-// (128 accumulators and a 2-chunk weight ring per wave).
-// * Each wave streams its own weight rows straight into registers through a
-//   kWideDepth-chunk ring (64 k per chunk; a lane's 16-byte fragment of the
-//   packed layout -- four contiguous 256-byte runs per instruction).
-// * The token rows (packed by the entry point into the workspace) are shared
-//   by all 8 waves: chunk by chunk, loaded straight into LDS (four buffers,
-//   two chunks ahead of use -- at least as far ahead as the weight ring, so
-//   that waiting for a chunk (the vector memory counter is in order) never
-//   waits for a weight chunk that is not due yet -- one
-//   barrier per chunk) in the packed order, so each 16-lane fragment read is
-//   one contiguous 256-byte run.
-// * Epilogue per group: bf16-rounded logits -> per-token best keys, merged
-//   into the wave's slot in LDS; at the end one key per token per workgroup,
-//   reduced across workgroups by argmax_reduce_kernel.
-// ---------------------------------------------------------------------------
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-constexpr int kWideWaves = 8;      // waves per workgroup (two per SIMD) = vocab tiles per group
-constexpr int kWideTokTiles = 8;   // 32-token tiles (M <= 256)
-constexpr int kWideChunk = 64;     // k per stage
-constexpr int kWideDepth = 2;      // weight chunks in flight per wave (two waves per SIMD: 256 registers)
-constexpr int kXBlocksPerWave = 32 / kWideWaves;  // 1 KiB blocks of a token-row chunk staged per wave
-constexpr int kUnroll = 8;         // stages per unrolled step: ring slot and LDS buffer fixed per position
-constexpr int kWideMaxGrid = 1024; // bound on the workgroups (sizes the workspace)
-constexpr int kWideMaxRows = 32 * kWideTokTiles;
-
-// s_waitcnt immediate (gfx9 encoding) waiting until at most `n` vector memory operations are outstanding,
-// with the other counters unconstrained: vmcnt bits [3:0] and [15:14], expcnt [6:4], lgkmcnt [11:8].
-constexpr int waitcnt_vm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
-
-__device__ __forceinline__ f32x16 mfma_32x32x16(const u32x4& a, const u32x4& b, const f32x16& c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
-                                                 0, 0);
-}
-
-// The TT token-row fragments of one k16 step from LDS: 16 bytes per lane at byte address a + 4096 tt,
-// all requested before one wait, in one asm block.  As inline asm the reads are invisible to the
-// compiler's tracking of the token-row loads into LDS; that tracking cannot tell across the loop's back
-// edge which load wrote a buffer, and would otherwise wait for every load in flight once per pass.
-// The counted waits and barriers around the reads already order them after those loads.
-template <int TT>
-__device__ __forceinline__ void lds_fragments(u32x4 (&x)[TT], uint32_t a);
-template <>
-__device__ __forceinline__ void lds_fragments<2>(u32x4 (&x)[2], uint32_t a) {
-  asm volatile(
-      "ds_read_b128 %0, %2\n\t"
-      "ds_read_b128 %1, %2 offset:4096\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(x[0]), "=&v"(x[1])
-      : "v"(a));
-}
-template <>
-__device__ __forceinline__ void lds_fragments<4>(u32x4 (&x)[4], uint32_t a) {
-  asm volatile(
-      "ds_read_b128 %0, %4\n\t"
-      "ds_read_b128 %1, %4 offset:4096\n\t"
-      "ds_read_b128 %2, %4 offset:8192\n\t"
-      "ds_read_b128 %3, %4 offset:12288\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3])
-      : "v"(a));
-}
-template <>
-__device__ __forceinline__ void lds_fragments<8>(u32x4 (&x)[8], uint32_t a) {
-  asm volatile(
-      "ds_read_b128 %0, %8\n\t"
-      "ds_read_b128 %1, %8 offset:4096\n\t"
-      "ds_read_b128 %2, %8 offset:8192\n\t"
-      "ds_read_b128 %3, %8 offset:12288\n\t"
-      "ds_read_b128 %4, %8 offset:16384\n\t"
-      "ds_read_b128 %5, %8 offset:20480\n\t"
-      "ds_read_b128 %6, %8 offset:24576\n\t"
-      "ds_read_b128 %7, %8 offset:28672\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]), "=&v"(x[4]), "=&v"(x[5]), "=&v"(x[6]), "=&v"(x[7])
-      : "v"(a));
-}
-
-// TT: 32-token tiles computed (2, 4 or 8; rows past M are padding whose results nobody reads).
-template <int K, int TT>
-__global__ __launch_bounds__(64 * kWideWaves) void lm_head_wide_kernel(const bf16_t* __restrict__ xp, int M,
-                                                                      const bf16_t* w, int64_t N,
-                                                                      bf16_t* __restrict__ logits, int64_t ldl,
-                                                                      uint64_t* __restrict__ best_out) {
-  constexpr int kChunks = K / kWideChunk;
-  static_assert(K % 128 == 0, "packed k steps are 128 wide");
-  // X chunk: token row tile t (16 tokens) x block i (32 k) at (2t + i) * 512 elements, lane order inside.
-  // Four buffers (stage s reads s % 4; chunks go in two stages ahead), as separate arrays so the compiler
-  // can tell a load into one from reads of another.
-  __shared__ bf16_t xs0[kWideTokTiles * 2 * 2 * 512], xs1[kWideTokTiles * 2 * 2 * 512];
-  __shared__ bf16_t xs2[kWideTokTiles * 2 * 2 * 512], xs3[kWideTokTiles * 2 * 2 * 512];
-  __shared__ uint64_t wave_best[kWideWaves][kWideMaxRows];
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n = lane & 31, h = lane >> 5, r = lane & 15;
-  const int x_tiles = (M + 15) / 16;             // packed 16-row token tiles present
-  const int64_t w_last = (N + 15) / 16 - 1;       // last packed 16-row weight tile
-  const int64_t nt32 = (N + 31) / 32;
-  const int64_t lo = (int64_t)blockIdx.x * nt32 / gridDim.x, hi = (int64_t)(blockIdx.x + 1) * nt32 / gridDim.x;
-  const int64_t groups = (hi - lo + kWideWaves - 1) / kWideWaves;
-  const int64_t stages = groups * kChunks;
-
-  for (int i = tid; i < kWideWaves * kWideMaxRows; i += 64 * kWideWaves) (&wave_best[0][0])[i] = 0;
-
-  // Weight fragment of stage s (group s / kChunks, chunk s % kChunks), k16 step kk: lane (n, h) holds
-  // W[32 vt + n][64 c + 16 kk + 8h, +8).  A wave without a vocab tile in a group (the last group of a
-  // range that is not a multiple of kWideWaves, or past the last stage) still issues the load, so every
-  // wave's counted waits hold, but reads the same offset in the first token-row tile (cached, in range:
-  // the offset is below 16 K) and computes nothing with it.
-  auto wfrag = [&](int64_t s, int kk) {
-    s = s < stages ? s : stages - 1;
-    const int64_t gi = s / kChunks;
-    const int c = (int)(s - gi * kChunks);
-    const int64_t vt = lo + gi * kWideWaves + wave;
-    int64_t t = 2 * vt + (n >> 4);
-    t = t < w_last ? t : w_last;
-    const int i = 2 * (c & 1) + (kk >> 1), g = 2 * (kk & 1) + h;
-    const int64_t inner = (c >> 1) * (16 * kKStep) + i * 512 + (16 * g + r) * 8;
-    return ld_w((vt < hi ? w + t * (K * 16) : xp) + inner);  // vt < hi is wave-uniform
-  };
-  // Token rows of chunk c straight into an LDS buffer (global_load_lds, 16 bytes per lane: lane i of an
-  // instruction writes bytes [16i, 16i + 16) of a 1 KiB block): 32 blocks (block j: token row tile j / 2,
-  // half j % 2 of the chunk's 64 k), kXBlocksPerWave per wave.  Tiles past the last one re-read it.
-  auto xdma = [&](int c, bf16_t* dst) {
-#pragma unroll
-    for (int u = 0; u < kXBlocksPerWave; ++u) {
-      const int j = kXBlocksPerWave * wave + u, t = j >> 1;
-      const int tl = t < x_tiles ? t : x_tiles - 1;
-      __builtin_amdgcn_global_load_lds(
-          (const void __attribute__((address_space(1)))*)(xp + (int64_t)tl * (K * 16) + (c >> 1) * (16 * kKStep) +
-                                                          (2 * (c & 1) + (j & 1)) * 512 + lane * 8),
-          (void __attribute__((address_space(3)))*)(dst + j * 512), 16, 0, 0);
-    }
-  };
-
-  u32x4 ring[kWideDepth][4];
-#pragma unroll
-  for (int d = 0; d < kWideDepth; ++d)
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) ring[d][kk] = wfrag(d, kk);
-  // Stage s's token rows go in at stage s - 2 (chunk c of stage s is s % kChunks; past the last stage the
-  // loads repeat a valid chunk into a buffer nobody reads), so every stage issues the same loads: its
-  // token-row block loads, then its 4 weight loads.  At the end of stage s, the loads issued after
-  // stage s + 1's token rows are 4 + (kXBlocksPerWave + 4); everything older has landed.
-  auto xchunk = [&](int64_t st) { return (int)((st < stages ? st : stages - 1) % kChunks); };
-  xdma(xchunk(0), xs0);
-  xdma(xchunk(1), xs1);
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm(kXBlocksPerWave));
-  __syncthreads();
-
-  f32x16 acc[TT];
-#pragma unroll
-  for (int tt = 0; tt < TT; ++tt)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[tt][e] = 0.f;
-
-  // Stage s = gi * kChunks + c: chunk c of group gi.  kChunks is a multiple of kWideDepth (even), so
-  // stage s uses ring slot s % kWideDepth and LDS buffer s % 2, both fixed per unrolled position.
-  static_assert(kChunks % kUnroll == 0 && kUnroll % kWideDepth == 0 && kUnroll % 4 == 0,
-                "ring slots and buffers must be static");
-  for (int64_t gi = 0; gi < groups; ++gi) {
-    // Waves without a vocab tile in this group skip the products (wave-uniform); their loads and
-    // barriers are the same as everyone's.
-    const bool active = lo + gi * kWideWaves + wave < hi;
-    for (int c0 = 0; c0 < kChunks; c0 += kUnroll) {
-#pragma unroll
-      for (int d = 0; d < kUnroll; ++d) {
-        const int c = c0 + d;
-        const int64_t s = gi * kChunks + c;
-        bf16_t* const bufs[4] = {xs0, xs1, xs2, xs3};
-        xdma(xchunk(s + 2), bufs[(d + 2) & 3]);  // read at stage s - 2, before the last barrier
-        __builtin_amdgcn_sched_barrier(0);
-        // This stage's weight chunk (loaded during stage s - 2) is in: the loads issued after it are stage
-        // s - 1's and this stage's token rows and stage s - 1's weights.
-        __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * kXBlocksPerWave + 4));
-        // Lane (n, h)'s fragment of token tile tt, k16 step kk: X[32 tt + n][64 c + 16 kk + 8h, +8) at element
-        // (4 tt + 2 (n / 16)) * 512 + (kk / 2) * 512 + (16 (2 (kk % 2) + h) + r) * 8 of the buffer.
-        const uint32_t xb = (uint32_t)(uintptr_t)bufs[d & 3] + 2048 * (n >> 4) + 16 * (16 * h + r);
-        if (active) {
-#pragma unroll
-          for (int kk = 0; kk < 4; ++kk) {
-            u32x4 xf[TT];
-            lds_fragments<TT>(xf, xb + 1024 * (kk >> 1) + 512 * (kk & 1));
-#pragma unroll
-            for (int tt = 0; tt < TT; ++tt) acc[tt] = mfma_32x32x16(ring[d % kWideDepth][kk], xf[tt], acc[tt]);
-          }
-        }
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) ring[d % kWideDepth][kk] = wfrag(s + kWideDepth, kk);
-        __builtin_amdgcn_sched_barrier(0);
-        // The only LDS data that crosses waves in the loop is what the token-row loads write, and the
-        // count above covers it; a barrier with fences (or __syncthreads) would also wait for every
-        // weight load in flight.  The memory clobber keeps LDS reads on their side of the barrier.
-        __builtin_amdgcn_s_waitcnt(waitcnt_vm(4 + (kXBlocksPerWave + 4)));  // a wait the compiler can count on
-        asm volatile("s_barrier" ::: "memory");
-      }
-    }
-    // Group epilogue: vocab tile vt of this wave; lane (n, h) holds logits of vocab rows
-    // 32 vt + 8 (e / 4) + 4h + e % 4 for token 32 tt + n.
-    const int64_t vt = lo + gi * kWideWaves + wave;
-    if (vt < hi) {  // wave-uniform
-#pragma unroll
-      for (int tt = 0; tt < TT; ++tt) {
-        const int tok = 32 * tt + n;
-        uint64_t best = 0;
-#pragma unroll
-        for (int m4 = 0; m4 < 4; ++m4) {
-          const int64_t col0 = 32 * vt + 8 * m4 + 4 * h;
-          uint32_t b16[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            b16[j] = f2bf(acc[tt][4 * m4 + j]);
-            if (col0 + j < N) {
-              const uint64_t key = argmax_key(b16[j] << 16, (uint32_t)(col0 + j));
-              best = key > best ? key : best;
-            }
-          }
-          if (logits && tok < M) {
-            bf16_t* dst = logits + (int64_t)tok * ldl + col0;
-            if (col0 + 3 < N) {
-              *reinterpret_cast<u32x2*>(dst) = u32x2{b16[0] | (b16[1] << 16), b16[2] | (b16[3] << 16)};
-            } else {
-              for (int j = 0; j < 4; ++j)
-                if (col0 + j < N) dst[j] = (bf16_t)b16[j];
-            }
-          }
-        }
-        const uint64_t o = shfl_xor_u64(best, 32);
-        best = o > best ? o : best;
-        if (h == 0 && best > wave_best[wave][tok]) wave_best[wave][tok] = best;
-      }
-    }
-#pragma unroll
-    for (int tt = 0; tt < TT; ++tt)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[tt][e] = 0.f;
-  }
-  __syncthreads();
-
-  if (tid < M) {
-    uint64_t b = 0;
-#pragma unroll
-    for (int wv = 0; wv < kWideWaves; ++wv) b = wave_best[wv][tid] > b ? wave_best[wv][tid] : b;
-    best_out[(int64_t)blockIdx.x * M + tid] = b;
-  }
-}
-
 // Workspace of the wide path: per-workgroup keys (at most kWideMaxGrid workgroups), then the packed token
 // rows (hidden size at most 2048).
 size_t wide_x_offset(int64_t m) { return ((size_t)kWideMaxGrid * (size_t)m * sizeof(uint64_t) + 255) / 256 * 256; }
@@ -792,26 +526,6 @@ size_t wide_workspace_bytes(int64_t m) { return wide_x_offset(m) + (size_t)((m +
 // Row counts and hidden sizes the wide LM head takes (packed weight only).
 bool lm_head_wide_supported(int64_t m, int64_t k, bool packed) {
   return packed && m > 32 && m <= kWideMaxRows && (k == 512 || k == 1024 || k == 2048);
-}
-
-template <int TT>
-int launch_lm_head_wide_tt(const bf16_t* xp, int M, const bf16_t* w, int64_t K, int64_t N, bf16_t* logits,
-                           uint64_t* best, int grid, hipStream_t s) {
-  const dim3 g((unsigned)grid), b(64 * kWideWaves);
-  switch (K) {
-    case 512: hipLaunchKernelGGL((lm_head_wide_kernel<512, TT>), g, b, 0, s, xp, M, w, N, logits, N, best); break;
-    case 1024: hipLaunchKernelGGL((lm_head_wide_kernel<1024, TT>), g, b, 0, s, xp, M, w, N, logits, N, best); break;
-    case 2048: hipLaunchKernelGGL((lm_head_wide_kernel<2048, TT>), g, b, 0, s, xp, M, w, N, logits, N, best); break;
-    default: return OXR_ERR_UNSUPPORTED;
-  }
-  return OXR_LAUNCH_STATUS();
-}
-
-int launch_lm_head_wide(const bf16_t* xp, int M, const bf16_t* w, int64_t K, int64_t N, bf16_t* logits,
-                        uint64_t* best, int grid, hipStream_t s) {
-  if (M <= 64) return launch_lm_head_wide_tt<2>(xp, M, w, K, N, logits, best, grid, s);
-  if (M <= 128) return launch_lm_head_wide_tt<4>(xp, M, w, K, N, logits, best, grid, s);
-  return launch_lm_head_wide_tt<8>(xp, M, w, K, N, logits, best, grid, s);
 }
 
 // Compute units of the current device (one persistent LM-head workgroup each).
