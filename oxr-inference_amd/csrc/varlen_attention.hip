@@ -380,22 +380,24 @@ constexpr int kPLoadsPerWave = kKeyTile * kVD * 2 / 1024 / kPWaves;
 template <bool kCausal>
 __global__ __launch_bounds__(64 * kPWaves, 1) void varlen_attention_pp_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
-    const int32_t* __restrict__ cu_seqlens, int H, int KV, int num_qtiles, int num_pairs, float scale_log2,
+    const int32_t* __restrict__ cu_seqlens, int H, int KV, int num_qtiles, int parts, float scale_log2,
     bf16_t* __restrict__ out) {
   __shared__ bf16_t s_k0[kKeyTile * kVD], s_k1[kKeyTile * kVD];
   __shared__ bf16_t s_v0[kKeyTile * kVD], s_v1[kKeyTile * kVD];
 
-  // Pairs are dealt to the XCDs in turn (workgroup b runs on XCD b % 8), each XCD taking its pairs one after
-  // another, so a pair's K/V stays in one L2 and every XCD gets heads of every sequence.  A contiguous eighth
-  // of the pairs per XCD gave the XCDs unequal lengths: 6 sequences of 1023 to 1914 tokens (16/8 heads) took
+  // Units -- a pair, or with KV no multiple of 8 one of the `parts` interleaved parts of its query tiles -- are
+  // dealt to the XCDs in turn (workgroup b runs on XCD b % 8), each XCD taking its units one after another.
+  // So a unit's K/V stays in one L2 and every XCD gets the same share of every sequence.  A contiguous eighth
+  // of the items per XCD gave the XCDs unequal lengths: 6 sequences of 1023 to 1914 tokens (16/8 heads) took
   // 185 us that way, 158 this way.  (Longest sequence first: 161.)
-  const int slot = (int)blockIdx.x >> 3;
-  const int pair = ((int)blockIdx.x & 7) + 8 * (slot / num_qtiles);
-  if (pair >= num_pairs) return;  // whole workgroup: before any barrier
+  const int per_unit = (num_qtiles + parts - 1) / parts, slot = (int)blockIdx.x >> 3;
+  const int unit = ((int)blockIdx.x & 7) + 8 * (slot / per_unit);
+  const int pair = unit / parts, qt = num_qtiles - 1 - (unit % parts + parts * (slot % per_unit));
+  if (qt < 0) return;  // whole workgroup: before any barrier
   const int seq = pair / KV, kvh = pair - seq * KV;
   const int start = cu_seqlens[seq], len = cu_seqlens[seq + 1] - start;
   const int G = H / KV, rph = kPRows / G;
-  const int q0 = (num_qtiles - 1 - slot % num_qtiles) * rph;
+  const int q0 = qt * rph;
   if (q0 >= len) return;  // whole workgroup: before any barrier
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -649,14 +651,14 @@ extern "C" int oxr_varlen_attention(const oxr_bf16* q, const oxr_bf16* k, const 
   // group, so the lists keep that much headroom below INT32_MAX.
   OXR_RETURN_IF((int64_t)num_qtiles * num_kv_heads * num_seqs > INT32_MAX - 8 * 8 * kPersistentSlots,
                 OXR_ERR_UNSUPPORTED);
-  // (The bidirectional grid, rounded up to 8 pairs, is below 2^32.)
   const float scale_log2 = scale * 1.4426950408889634f;
   hipStream_t s = (hipStream_t)stream;
   const int num_pairs = num_seqs * num_kv_heads;
   if (!causal) {
-    const dim3 grid((unsigned)(8 * ((num_pairs + 7) / 8) * num_qtiles));
+    const int parts = num_kv_heads % 8 == 0 ? 1 : num_kv_heads % 4 == 0 ? 2 : num_kv_heads % 2 == 0 ? 4 : 8;
+    const dim3 grid((unsigned)num_pairs * parts * ((num_qtiles + parts - 1) / parts));
     hipLaunchKernelGGL(varlen_attention_pp_kernel<false>, grid, dim3(64 * kPWaves), 0, s, q, k, v, cu_seqlens,
-                       num_heads, num_kv_heads, num_qtiles, num_pairs, scale_log2, out);
+                       num_heads, num_kv_heads, num_qtiles, parts, scale_log2, out);
   } else {
     // Two workgroups per CU, or fewer when the largest XCD group has fewer items.
     static std::atomic<uint32_t> launches{0};
