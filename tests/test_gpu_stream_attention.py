@@ -1,0 +1,105 @@
+"""Paged attention of large batches, whose contexts are cut into equal shares of the whole batch's keys
+(256 or more (context, kv-head group) units): contexts inside one share, over several, starting exactly on a
+share, empty, of one key, and one far longer than the rest; every head grouping, both page sizes, verify and
+decode widths -- against a float64 softmax over the gathered keys, and the fused launch against the separate
+q/k norm + RoPE + store and attention calls bit for bit.  Tolerance: the outputs' bf16 rounding (2^-9) and the
+bf16 rounding of the probabilities (2^-9 of a convex combination of |v| <= 6).
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import announce, pkg
+
+pytestmark = pytest.mark.gpu
+attention = pkg("attention")
+kernels = pkg("kernels")
+
+D = 128
+
+
+def _batch(lens: list[int], bs: int, kv: int, g: torch.Generator):
+    pages = [-(-max(n, 1) // bs) for n in lens]
+    order = np.random.default_rng(len(lens)).permutation(sum(pages)).astype(np.int32)
+    table = np.zeros((len(lens), max(pages)), dtype=np.int32)
+    at = 0
+    for b, n in enumerate(pages):
+        table[b, :n] = order[at:at + n]
+        at += n
+    shape = (sum(pages), bs, kv, D)
+    kc = torch.randn(shape, generator=g, device="cuda").clamp(-6, 6).to(torch.bfloat16)
+    vc = torch.randn(shape, generator=g, device="cuda").clamp(-6, 6).to(torch.bfloat16)
+    return kc, vc, torch.from_numpy(table).cuda(), torch.tensor(lens, dtype=torch.int32, device="cuda")
+
+
+def _check(out: torch.Tensor, q: torch.Tensor, kc, vc, table, lens: list[int]) -> None:
+    _, s, h, _ = q.shape
+    kv, bs = kc.shape[2], kc.shape[1]
+    for b, n in enumerate(lens):
+        if n < s:
+            continue
+        at = torch.arange(n, device="cuda")
+        slot = table[b].long()[at // bs] * bs + at % bs
+        k, v = (c.view(-1, kv, D)[slot].double().repeat_interleave(h // kv, 1) for c in (kc, vc))
+        scores = (q[b].double()[:, :, None, :] * 1.0).permute(1, 0, 2, 3).squeeze(2) @ k.permute(1, 2, 0).contiguous()
+        scores = scores * D ** -0.5
+        scores.masked_fill_(at[None, :] > (n - s + torch.arange(s, device="cuda"))[:, None], float("-inf"))
+        want = (torch.softmax(scores, -1) @ v.permute(1, 0, 2).contiguous()).permute(1, 0, 2)
+        mass = (torch.softmax(scores, -1) @ v.abs().permute(1, 0, 2).contiguous()).permute(1, 0, 2)
+        err = (out[b].double() - want).abs()
+        assert bool((err <= 2.0 ** -8 * want.abs() + 2.0 ** -8 * mass + 1e-5).all()), (b, n, err.max().item())
+
+
+MIXED = [1, 3000, 32, 33, 0, 700, 4096, 2, 1024, 513] + [64 + 37 * i for i in range(60)]
+
+
+@pytest.mark.parametrize("s,h,kv,bs", [(1, 16, 8, 256), (1, 16, 8, 16), (4, 16, 8, 16), (8, 16, 8, 256), (1, 16, 4, 16),
+                                       (1, 32, 4, 16), (2, 8, 8, 256), (3, 5, 5, 16), (1, 128, 8, 16)])
+def test_mixed_contexts(s: int, h: int, kv: int, bs: int) -> None:
+    g = torch.Generator(device="cuda").manual_seed(s * 100 + h + kv)
+    lens = (MIXED * 2)[: max(70, 256 // max(kv // 2, 1))]
+    kc, vc, table, lens_t = _batch(lens, bs, kv, g)
+    q = torch.randn(len(lens), s, h, D, generator=g, device="cuda").to(torch.bfloat16)
+    announce("stream attention", s, h, kv, bs, len(lens))
+    out = attention.paged_extend(q, kc, vc, lens_t, table)
+    torch.cuda.synchronize()
+    _check(out, q, kc, vc, table, lens)
+
+
+@pytest.mark.parametrize("lens", [[1024] * 64, [544] * 128, [16] * 63 + [8000], [600] * 256, [513] * 64 + [1] * 64])
+def test_equal_long_and_short_contexts(lens: list[int]) -> None:
+    """Shares that end exactly between contexts, one context that fills many shares, more contexts than shares."""
+    g = torch.Generator(device="cuda").manual_seed(len(lens))
+    kc, vc, table, lens_t = _batch(lens, 16, 8, g)
+    q = torch.randn(len(lens), 1, 16, D, generator=g, device="cuda").to(torch.bfloat16)
+    announce("stream lengths", lens[0], lens[-1], len(lens))
+    out = attention.paged_extend(q, kc, vc, lens_t, table)
+    torch.cuda.synchronize()
+    _check(out, q, kc, vc, table, lens)
+
+
+@pytest.mark.parametrize("s,h,kv", [(1, 16, 8), (4, 16, 8), (8, 16, 8), (3, 8, 8)])
+def test_fused_equals_separate_calls(s: int, h: int, kv: int) -> None:
+    """Contexts of at least s keys whose new tokens straddle shares; output and both caches."""
+    g = torch.Generator(device="cuda").manual_seed(s)
+    lens = [max(n, s) for n in MIXED] + [256] * 10
+    kc, vc, table, lens_t = _batch(lens, 16, kv, g)
+    n = len(lens) * s
+    qkv = torch.randn(n, (h + 2 * kv) * D, generator=g, device="cuda").to(torch.bfloat16)
+    qw, kw = ((0.5 + torch.rand(D, generator=g, device="cuda")).to(torch.bfloat16) for _ in range(2))
+    angles = torch.rand(max(lens), D // 2, generator=g, device="cuda") * 6.28
+    cos, sin = angles.cos().to(torch.bfloat16), angles.sin().to(torch.bfloat16)
+    pos = (lens_t.long()[:, None] - s + torch.arange(s, device="cuda")).reshape(-1)
+    slots = table.long().gather(1, pos.view(-1, s) // 16).view(-1) * 16 + pos % 16
+    k2, v2 = kc.clone(), vc.clone()
+    announce("stream fused", s, h, kv)
+    q, _, _ = kernels.qk_norm_rope_store(qkv, qw, kw, cos[pos].contiguous(), sin[pos].contiguous(), 1e-6, k2, v2, slots,
+                                         h, kv, D, need_kv=False)
+    want = attention.paged_extend(q.view(len(lens), s, h, D), k2, v2, lens_t, table)
+    got = attention.qk_norm_rope_paged_extend(qkv, qw, kw, cos, sin, pos, 1e-6, kc, vc, slots, lens_t, table, h)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    assert torch.equal(kc.view(torch.int16), k2.view(torch.int16)) and torch.equal(vc, v2)
