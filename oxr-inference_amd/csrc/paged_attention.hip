@@ -237,27 +237,28 @@ __device__ __forceinline__ void stream_split(StreamSplit& sp, const int32_t* __r
 // JR: rounds of the fused prologue's 32 row jobs (HPW * (R + 2 S) <= 32 * JR).
 // kPlanned: pieces from a plan (paged_extend_plan_kernel); otherwise `splits` even pieces per context.
 // kStream: the batch's contexts end to end, cut into `splits` equal shares of 32-key units (StreamSplit);
-// workgroup blockIdx.x takes the pieces of contexts in its share one after another.
-// W: waves per workgroup.
-template <bool kFused, int HPW, int NT, int JR, bool kPlanned, bool kStream = false, int W = kWaves>
-__global__ __launch_bounds__(64 * W, W == kWaves ? 1 : 2) void paged_extend_kernel(
+// workgroup (head group, share) takes the pieces of contexts in its share one after another.  (Head groups
+// are neighbours in dispatch order: they read neighbouring slices of the same token rows.)
+template <bool kFused, int HPW, int NT, int JR, bool kPlanned, bool kStream = false>
+__global__ __launch_bounds__(64 * kWaves) void paged_extend_kernel(
     const bf16_t* __restrict__ q, const bf16_t* k_cache, const bf16_t* v_cache, const int32_t* __restrict__ seq_lens,
     const int32_t* __restrict__ block_table, int64_t table_stride, int S, int H, int KV, int log2_bs,
     int64_t num_blocks, float scale_log2, int max_seq_len, int splits, const int32_t* __restrict__ plan,
     float* __restrict__ part_o, float* __restrict__ part_ml, bf16_t* __restrict__ out, int out_packed, RopeArgs ra,
     int batch) {
-  constexpr int kStreams = W / HPW;  // waves per kv head
+  constexpr int kStreams = kWaves / HPW;  // waves per kv head
   // Two row tiles' q fragments (32 registers) would not fit next to two tiles'
   // accumulators and the two pair buffers: with NT = 2 the MFMAs read them from LDS.
   constexpr bool kQinLds = NT == 2;
-  __shared__ float s_o[W][16][kD];   // per wave: the K/V exchange buffer, then one row tile's results
+  __shared__ float s_o[kWaves][16][kD];   // per wave: the K/V exchange buffer, then one row tile's results
   __shared__ u32x4 s_q[kFused || kQinLds ? HPW : 1][kFused || kQinLds ? 16 * NT : 1][kD / 8];
   __shared__ u32x4 s_newk[kFused ? HPW : 1][kFused ? kMaxNew : 1][kD / 8];
   __shared__ u32x4 s_newv[kFused ? HPW : 1][kFused ? kMaxNew : 1][kD / 8];
-  __shared__ float s_m[W][16], s_l[W][16];
+  __shared__ float s_m[kWaves][16], s_l[kWaves][16];
   __shared__ int s_pages[kMaxSpanPages];
 
   const int G = H / KV, R = S * G;
+  const int head_group = kStream ? blockIdx.x : blockIdx.y;  // kv heads [HPW * head_group, +HPW)
 
   // One piece: keys [stream_begin, stream_end) of sequence b (kStream, partial unit `split`), else piece `split`.
   auto run_piece = [&](const int b, const int split, const int pieces, const bool use_plan, const int stream_len,
@@ -268,10 +269,10 @@ __global__ __launch_bounds__(64 * W, W == kWaves ? 1 : 2) void paged_extend_kern
   const int lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);  // wave-uniform, so its addressing is scalar
   const int r = lane & 15, g = lane >> 4;
-  // The workgroup owns kv heads [HPW * blockIdx.y, +HPW): wave w serves head
+  // The workgroup owns kv heads [HPW * head_group, +HPW): wave w serves head
   // slot w % HPW and walks that head's keys as stream w / HPW of kStreams.
   const int hs = wave % HPW, stream = wave / HPW;
-  const int kvh = (int)blockIdx.y * HPW + hs;
+  const int kvh = head_group * HPW + hs;
 
   // Fused: HPW * (R + 2S) row jobs of one 128-element row each, on 16 lanes, in
   // JR rounds of 32 -- per head slot, q rows [0, R), then the K rows and the V
@@ -295,12 +296,12 @@ __global__ __launch_bounds__(64 * W, W == kWaves ? 1 : 2) void paged_extend_kern
   if constexpr (kFused) {
 #pragma unroll
     for (int jr = 0; jr < JR; ++jr) {
-      const int job = (tid >> 4) + 4 * W * jr;
+      const int job = (tid >> 4) + kJobSlots * jr;
       f_valid[jr] = job < HPW * f_per_head;
       const int jv = f_valid[jr] ? job : 0;
       f_hs[jr] = jv / f_per_head;
       f_jj[jr] = jv % f_per_head;
-      const int kvh_j = (int)blockIdx.y * HPW + f_hs[jr];
+      const int kvh_j = head_group * HPW + f_hs[jr];
       int head;
       if (f_jj[jr] < R) {
         f_ss[jr] = f_jj[jr] / G;
@@ -383,7 +384,7 @@ __global__ __launch_bounds__(64 * W, W == kWaves ? 1 : 2) void paged_extend_kern
   // (Every thread writes its entry, past npages too -- never read -- so the
   // load above is not moved into a branch.)
   s_pages[tid] = (int)my_page;
-  for (int i = tid + 64 * W; i < npages; i += 64 * W) {  // spans beyond 512 pages
+  for (int i = tid + 64 * kWaves; i < npages; i += 64 * kWaves) {  // spans beyond 512 pages
     s_pages[i] = table_row[page0 + i];
   }
 
@@ -404,7 +405,7 @@ __global__ __launch_bounds__(64 * W, W == kWaves ? 1 : 2) void paged_extend_kern
         else s_newv[f_hs[jr]][f_ss[jr]][f_s16] = f_raw[jr];
         const int pos = L - S + f_ss[jr];
         if (pos >= t_begin && pos < t_end && f_slot[jr] >= 0 && f_slot[jr] < ra.num_slots) {
-          const int kvh_j = (int)blockIdx.y * HPW + f_hs[jr];
+          const int kvh_j = head_group * HPW + f_hs[jr];
           bf16_t* dst = (is_k ? ra.k_store : ra.v_store) + (f_slot[jr] * KV + kvh_j) * kD + f_s16 * 8;
           st128(dst, is_k ? normed : f_raw[jr]);
         }
@@ -591,10 +592,10 @@ __global__ __launch_bounds__(64 * W, W == kWaves ? 1 : 2) void paged_extend_kern
     }
     __syncthreads();
     const int rows = min(16, R - 16 * t);
-    for (int idx = tid; idx < HPW * rows * (kD / 4); idx += 64 * W) {
+    for (int idx = tid; idx < HPW * rows * (kD / 4); idx += 64 * kWaves) {
       const int ho = idx / (rows * (kD / 4)), rl = (idx / (kD / 4)) % rows, d0 = (idx % (kD / 4)) * 4;
       const int rr = 16 * t + rl;
-      const int kvh_o = (int)blockIdx.y * HPW + ho;
+      const int kvh_o = head_group * HPW + ho;
       // Even: the (sequence, piece) unit; planned: this workgroup's own slot (the plan maps pieces to slots).
       const int64_t unit = kStream    ? (int64_t)kvh_o * 2 * splits + split
                            : use_plan ? ((int64_t)blockIdx.z * KV + kvh_o) * splits + blockIdx.x
@@ -630,8 +631,8 @@ __global__ __launch_bounds__(64 * W, W == kWaves ? 1 : 2) void paged_extend_kern
 
   if constexpr (kStream) {
     __shared__ StreamSplit sp;
-    stream_split<64 * W>(sp, seq_lens, batch, max_seq_len, splits);
-    const int slot = blockIdx.x;
+    stream_split<64 * kWaves>(sp, seq_lens, batch, max_seq_len, splits);
+    const int slot = blockIdx.y;
     if (sp.whole) {
       if (slot < batch) run_piece(slot, 0, 0, false, sp.len[slot], 0, sp.len[slot]);
       return;
@@ -1004,23 +1005,30 @@ size_t partial_bytes(int32_t batch, int32_t num_kv_heads, int32_t max_seq_len) {
   return partial_units(batch, num_kv_heads, max_seq_len) * kPartRows * (kD + 2) * sizeof(float);
 }
 
-// A kStream launch: two 4-wave workgroups per CU, kv heads per workgroup and shares; no shares: one 8-wave
-// workgroup per context and head group instead.  Streams take over where that would be the launch, at 256 or
-// more (context, head group) units: contexts of different lengths then leave CUs idle behind the longest (a
-// workgroup streams at most 50 GB/s), and nothing covers a workgroup's fixed 8 us.  Below, contexts are split
-// evenly or by a plan.  Two heads only while their row jobs fit one round (two rounds spill).  The partials
-// (two units of R rows a share) fit the workspace of the batch; up to 512 keys there is nothing to share.
+// A kStream launch: kv heads per workgroup and shares (one workgroup per CU); no shares: a workgroup per context
+// and head group instead.  Streams take over where that would be the launch and would fill the chip less than
+// twice, at 256 to 479 (context, head group) units: there contexts of different lengths leave CUs idle behind
+// the longest (a workgroup streams at most 50 GB/s).  Decode, 16/8 heads, us, without and with: 64 contexts of
+// 256-8192 keys 226 / 199, 96 of 200-3000 165 / 125; 64 of about 2020 keys 89 / 92 (the merge launch finds
+// nothing to do); 128 of 200-3000, 8/8 heads, two rounds of workgroups: 170 / 173.  Two 4-wave workgroups per
+// CU: 203 and 105 for the first and third.  Below 256 units contexts are split evenly or by a plan.  The
+// partials (two units of R rows a share) fit the workspace of the batch.  Contexts of up to 1024 keys are too
+// short to share: 64 of 500-600 keys 30 / 34.
+constexpr int kMinStreamKeys = 1024;
+constexpr int kMaxStreamUnits = 480;
 struct StreamLaunch {
   int hpw, shares;
 };
 StreamLaunch stream_launch(int32_t batch, int32_t tokens_per_seq, int32_t num_heads, int32_t num_kv_heads,
                            int32_t max_seq_len, int splits) {
   const int rows = tokens_per_seq * (num_heads / num_kv_heads);
-  const int jobs = tokens_per_seq * (num_heads / num_kv_heads + 2);  // per head; 16 a round
-  if (splits != 1 || batch > kStreamMaxBatch || rows > 16 || jobs > kJobSlots || max_seq_len <= 512) return {1, 0};
-  const int hpw = num_kv_heads % 2 == 0 && 2 * jobs <= 16 ? 2 : 1;
+  const int jobs = tokens_per_seq * (num_heads / num_kv_heads + 2);  // per head
+  const int hpw = num_kv_heads % 2 == 0 && 2 * jobs <= kJobSlots ? 2 : 1;
+  if (splits != 1 || batch > kStreamMaxBatch || rows > 16 || jobs > kJobSlots || max_seq_len <= kMinStreamKeys ||
+      batch * (num_kv_heads / hpw) >= kMaxStreamUnits)
+    return {1, 0};
   const int64_t room = (int64_t)partial_units(batch, num_kv_heads, max_seq_len) * kPartRows;
-  const int64_t shares = std::min<int64_t>(512 / (num_kv_heads / hpw), room / (2 * (int64_t)num_kv_heads * rows));
+  const int64_t shares = std::min<int64_t>(256 / (num_kv_heads / hpw), room / (2 * (int64_t)num_kv_heads * rows));
   return {hpw, shares >= 16 ? (int)shares : 0};
 }
 
@@ -1073,20 +1081,17 @@ int launch_paged_extend(const oxr_bf16* q, const oxr_bf16* k_cache, const oxr_bf
     const RopeArgs rope = ra ? *ra : RopeArgs{};
     const float scale_log2 = scale * 1.4426950408889634f;
     auto launch = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3(std::max(shares, (int)batch), num_kv_heads / st.hpw), dim3(64 * 4), 0, s,
+      hipLaunchKernelGGL(kernel, dim3(num_kv_heads / st.hpw, std::max(shares, (int)batch)), dim3(64 * kWaves), 0, s,
                          ra ? nullptr : q, k_cache, v_cache, seq_lens, block_table, table_stride, tokens_per_seq,
                          num_heads, num_kv_heads, log2_bs, num_blocks, scale_log2, max_seq_len, shares, nullptr,
                          part_o, part_ml, out, out_packed, rope, batch);
     };
     if (!ra) {
-      if (st.hpw == 2) launch(paged_extend_kernel<false, 2, 1, 1, false, true, 4>);
-      else launch(paged_extend_kernel<false, 1, 1, 1, false, true, 4>);
-    } else if (st.hpw == 2) {
-      launch(paged_extend_kernel<true, 2, 1, 1, false, true, 4>);
-    } else if (tokens_per_seq * (num_heads / num_kv_heads + 2) <= 16) {
-      launch(paged_extend_kernel<true, 1, 1, 1, false, true, 4>);
+      if (st.hpw == 2) launch(paged_extend_kernel<false, 2, 1, 1, false, true>);
+      else launch(paged_extend_kernel<false, 1, 1, 1, false, true>);
     } else {
-      launch(paged_extend_kernel<true, 1, 1, 2, false, true, 4>);
+      if (st.hpw == 2) launch(paged_extend_kernel<true, 2, 1, 1, false, true>);
+      else launch(paged_extend_kernel<true, 1, 1, 1, false, true>);
     }
     const int status = OXR_LAUNCH_STATUS();
     if (status) return status;

@@ -1,5 +1,5 @@
 """Paged attention of large batches, whose contexts are cut into equal shares of the whole batch's keys
-(256 or more (context, kv-head group) units): contexts inside one share, over several, starting exactly on a
+(256 to 479 (context, kv-head group) units): contexts inside one share, over several, starting exactly on a
 share, empty, of one key, and one far longer than the rest; every head grouping, both page sizes, verify and
 decode widths -- against a float64 softmax over the gathered keys, and the fused launch against the separate
 q/k norm + RoPE + store and attention calls bit for bit.  Tolerance: the outputs' bf16 rounding (2^-9) and the
@@ -53,6 +53,12 @@ def _check(out: torch.Tensor, q: torch.Tensor, kc, vc, table, lens: list[int]) -
         assert bool((err <= 2.0 ** -8 * want.abs() + 2.0 ** -8 * mass + 1e-5).all()), (b, n, err.max().item())
 
 
+def _sequences(s: int, h: int, kv: int) -> int:
+    """A batch of just over 256 units: head groups of two kv heads while their rows fit, else one."""
+    groups = kv // 2 if kv % 2 == 0 and 2 * s * (h // kv + 2) <= 32 else kv
+    return -(-256 // groups) + 6
+
+
 MIXED = [1, 3000, 32, 33, 0, 700, 4096, 2, 1024, 513] + [64 + 37 * i for i in range(60)]
 
 
@@ -60,7 +66,7 @@ MIXED = [1, 3000, 32, 33, 0, 700, 4096, 2, 1024, 513] + [64 + 37 * i for i in ra
                                        (1, 32, 4, 16), (2, 8, 8, 256), (3, 5, 5, 16), (1, 128, 8, 16)])
 def test_mixed_contexts(s: int, h: int, kv: int, bs: int) -> None:
     g = torch.Generator(device="cuda").manual_seed(s * 100 + h + kv)
-    lens = (MIXED * 2)[: max(70, 256 // max(kv // 2, 1))]
+    lens = (MIXED * 4)[: _sequences(s, h, kv)]
     kc, vc, table, lens_t = _batch(lens, bs, kv, g)
     q = torch.randn(len(lens), s, h, D, generator=g, device="cuda").to(torch.bfloat16)
     announce("stream attention", s, h, kv, bs, len(lens))
@@ -69,7 +75,7 @@ def test_mixed_contexts(s: int, h: int, kv: int, bs: int) -> None:
     _check(out, q, kc, vc, table, lens)
 
 
-@pytest.mark.parametrize("lens", [[1024] * 64, [544] * 128, [16] * 63 + [8000], [600] * 256, [513] * 64 + [1] * 64])
+@pytest.mark.parametrize("lens", [[1024] * 64, [1056] * 100, [16] * 63 + [8000], [600] * 110 + [1100], [1025] * 60 + [1] * 59])
 def test_equal_long_and_short_contexts(lens: list[int]) -> None:
     """Shares that end exactly between contexts, one context that fills many shares, more contexts than shares."""
     g = torch.Generator(device="cuda").manual_seed(len(lens))
@@ -85,7 +91,7 @@ def test_equal_long_and_short_contexts(lens: list[int]) -> None:
 def test_fused_equals_separate_calls(s: int, h: int, kv: int) -> None:
     """Contexts of at least s keys whose new tokens straddle shares; output and both caches."""
     g = torch.Generator(device="cuda").manual_seed(s)
-    lens = [max(n, s) for n in MIXED] + [256] * 10
+    lens = [max(n, s) for n in (MIXED * 4)[: _sequences(s, h, kv)]]
     kc, vc, table, lens_t = _batch(lens, 16, kv, g)
     n = len(lens) * s
     qkv = torch.randn(n, (h + 2 * kv) * D, generator=g, device="cuda").to(torch.bfloat16)
