@@ -73,6 +73,17 @@ __device__ __forceinline__ f32x16 mfma_32x32x16(const u32x4& a, const u32x4& b, 
                                                  0, 0);
 }
 
+// One 1 KiB block from memory into LDS (lane i's 16 bytes to lds + 16 i), as inline asm: the compiler's
+// counters do not see it, so LDS reads are scheduled without waits for blocks in flight; the counted waits
+// and barriers of the tile loop order them.  (s_nop: wait states between the scalar writes and their use.)
+__device__ __forceinline__ void dma_block(const char* base, uint32_t offset, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base)
+               : "memory");
+}
+__device__ __forceinline__ uint32_t lds_address(const bf16_t* p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) bf16_t*)p;
+}
+
 // LDS transpose read (gfx950 ds_read_b64_tr_b16).  Within each group of 16 lanes,
 // lane 4a + b receives element b of the 4 bf16 addressed by lanes a, a + 4,
 // a + 8 and a + 12 of its group, in that order.
@@ -144,22 +155,23 @@ __device__ __forceinline__ void varlen_item(const bf16_t* __restrict__ q, const 
   const int key_end = min(len, q0 + rph);  // keys this workgroup needs
   const int tiles = (key_end + kKeyTile - 1) / kKeyTile;
 
-  // Key tiles go straight from memory to LDS (global_load_lds, 16 bytes per lane: lane i of an
-  // instruction writes bytes [16i, 16i + 16) of a 1 KiB block, i.e. 4 rows of 256 bytes).  Rows
-  // are stored without padding, their 16-byte chunks rotated instead: K row r holds chunk c at
-  // position (c + r) mod 16, V row r at (c + 4r) mod 16.  That gives every fragment read below the
-  // banks of a 68-dword (K) or 80-dword (V) row pitch, the ones measured free of conflicts for
+  // Key tiles go straight from memory to LDS (lane i of a load writes bytes [16i, 16i + 16) of a 1 KiB block,
+  // i.e. 4 rows of 256 bytes).  Rows are stored without padding, their 16-byte chunks rotated instead: K row r
+  // holds chunk c at position (c + r) mod 16, V row r at (c + 4r) mod 16.  That gives every fragment read
+  // below the banks of a 68-dword (K) or 80-dword (V) row pitch, the ones measured free of conflicts for
   // these patterns.  Keys past the sequence re-read its last key (their scores are masked).
-  auto dma = [&](const bf16_t* src, int t, bf16_t* dst, int rot) {
+  const int64_t row_bytes = (int64_t)KV * kVD * 2;
+  const char* const kbase = (const char*)(k + ((int64_t)start * KV + kvh) * kVD);
+  const char* const vbase = (const char*)(v + ((int64_t)start * KV + kvh) * kVD);
+  auto dma = [&](const char* base, int t, const bf16_t* dst, int rot) __attribute__((always_inline)) {
+    const char* const tile = base + t * kKeyTile * row_bytes;
+    const int last = len - 1 - t * kKeyTile;  // the sequence's last key, in the tile
 #pragma unroll
     for (int u = 0; u < kLoadsPerWave; ++u) {
       const int j = kLoadsPerWave * wave + u;  // 1 KiB block: rows 4j .. 4j + 3
       const int row = 4 * j + (lane >> 4), pos = lane & 15;
-      const int key = min(t * kKeyTile + row, len - 1);
-      const int64_t base = ((int64_t)(start + key) * KV + kvh) * kVD;
-      __builtin_amdgcn_global_load_lds(
-          (const void __attribute__((address_space(1)))*)(src + base + 8 * ((pos - rot * row) & 15)),
-          (void __attribute__((address_space(3)))*)(dst + 512 * j), 16, 0, 0);
+      const uint32_t off = (uint32_t)min(row, last) * (uint32_t)row_bytes + 16 * ((pos - rot * row) & 15);
+      dma_block(tile, off, lds_address(dst) + 1024 * j);
     }
   };
 
@@ -180,47 +192,65 @@ __device__ __forceinline__ void varlen_item(const bf16_t* __restrict__ q, const 
   for (int dt = 0; dt < 4; ++dt)
     tr_off[dt] = 8 * ((4 * dt + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1) + 4 * tr_key) & 15) + 4 * (lane & 1);
 
-  // Raw scores of one tile: sv[kb][v] is key 32kb + 8(v/4) + 4h + v%4 of the tile for query n.  The
-  // two key blocks' chains alternate, so consecutive products are independent.
-  auto qk = [&](const bf16_t* kb_, f32x16 (&sv)[2]) {
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) sv[kb][e] = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        const u32x4 kf = *reinterpret_cast<const u32x4*>(kb_ + (32 * kb + n) * kVD + 8 * ((2 * i + h + n) & 15));
-        sv[kb] = mfma_32x32x16(kf, qf[i], sv[kb]);
-      }
-  };
-
-  // Tile t, software-pipelined by one tile: its scores `cur` were computed during tile t - 1; the
-  // products for tile t + 1's scores `nxt` (K in kq) are issued among this tile's exponentials, so
-  // the matrix cores work while the softmax runs on the vector unit.  K runs one tile ahead of V in
-  // the double buffers: tile t prefetches K(t + 2) into kd and V(t + 1) into vd, the buffers read
-  // during tile t - 1.  Past the last tile `nxt` is computed from a stale buffer and never used.
-  auto step = [&](int t, f32x16 (&cur)[2], f32x16 (&nxt)[2], const bf16_t* kq, const bf16_t* vp_, bf16_t* kd,
-                  bf16_t* vd) {
-    if (t + 2 < tiles) dma(k, t + 2, kd, 1);
-    if (t + 1 < tiles) dma(v, t + 1, vd, 4);
+  // Tile t: S^T = K Q^T, softmax, O^T += V^T P^T, with the LDS fragments read ahead of their products (K two
+  // dim steps, V one key step; a scheduling barrier per step) and each key step's exponentials behind the
+  // products of the step before.  Left to itself the compiler reads each K fragment right before its product
+  // and waits for the LDS 16 times a tile.  Earlier the registers of the read-ahead held the scores of tile
+  // t + 1, computed among tile t's exponentials; the other wave of the SIMD fills that gap as well.
+  // The next tile's blocks are requested first and have the whole tile to land.
+  auto step = [&](int t, const bf16_t* kb_, const bf16_t* vb, const bf16_t* kd, const bf16_t* vd)
+                  __attribute__((always_inline)) {
+    if (t + 1 < tiles) {
+      dma(kbase, t + 1, kd, 1);
+      dma(vbase, t + 1, vd, 4);
+    }
     const int kt0 = t * kKeyTile;
     if (kt0 <= wave_last) {  // wave-uniform: otherwise every key of this and later tiles is masked
+      auto kread = [&](int i, u32x4 (&d)[2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+          d[kb] = *reinterpret_cast<const u32x4*>(kb_ + (32 * kb + n) * kVD + 8 * ((2 * i + h + n) & 15));
+      };
+      auto vread = [&](int ks, u32x2 (&d)[4][2]) __attribute__((always_inline)) {
+        const bf16_t* vrow = vb + (16 * ks + tr_key) * kVD;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+          d[dt][0] = lds_read_tr16(vrow + tr_off[dt]);            // keys 16ks + 4h + (0..3)
+          d[dt][1] = lds_read_tr16(vrow + 8 * kVD + tr_off[dt]);  // keys 16ks + 8 + 4h + (0..3)
+        }
+      };
+      // sv[kb][v] is the raw score of key 32kb + 8(v/4) + 4h + v%4 of the tile for query n.
+      f32x16 sv[2];
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sv[kb][e] = 0.f;
+      u32x4 kr[3][2];
+      u32x2 vr[2][4][2];
+      kread(0, kr[0]);
+      kread(1, kr[1]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (i + 2 < 8) kread(i + 2, kr[(i + 2) % 3]);
+        if (i == 7) vread(0, vr[0]);
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) sv[kb] = mfma_32x32x16(kr[i % 3][kb], qf[i], sv[kb]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       // wave-uniform: a tile crossing the diagonal of one of the wave's rows, or the sequence end
       const bool edge = kt0 + kKeyTile - 1 > wave_first || kt0 + kKeyTile > len;
       if (edge) {
+        const int lim = min(len - 1, qpos) - kt0 - 4 * h;  // largest visible key, less the lane's 4h
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            const int key = kt0 + 32 * kb + 8 * (e >> 2) + 4 * h + (e & 3);
-            if (key >= len || key > qpos) cur[kb][e] = -INFINITY;
-          }
+          for (int e = 0; e < 16; ++e)
+            if (32 * kb + 8 * (e >> 2) + (e & 3) > lim) sv[kb][e] = -INFINITY;
       }
       // Row maximum (exact in any order) as a tree of three-input maxima (v_max3_f32): 32 scores in
       // 16 instructions instead of 31.
-      const float mx = xor32_max(row_max32(cur));
+      const float mx = xor32_max(row_max32(sv));
       const bool moved = mx > m_run;
       if (__builtin_amdgcn_ballot_w64(moved)) {
         const float m_new = moved ? mx : m_run;
@@ -232,55 +262,51 @@ __device__ __forceinline__ void varlen_item(const bf16_t* __restrict__ q, const 
         m_run = m_new;
         mc_run = mc_new;
       }
-      qk(kq, nxt);
       // P^T for key step ks: accumulators 8 (ks % 2) .. +7 of key block ks / 2, in k-slot order.
       // The tile's probabilities are summed as a tree, then added to the running sum.
-      u32x4 pb[4];
       float ps[16];
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
+      auto probabilities = [&](int ks) __attribute__((always_inline)) {
         float pv[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e)
-          pv[e] = __builtin_amdgcn_exp2f(fmaf(cur[ks >> 1][8 * (ks & 1) + e], scale_log2, -mc_run));
+          pv[e] = __builtin_amdgcn_exp2f(fmaf(sv[ks >> 1][8 * (ks & 1) + e], scale_log2, -mc_run));
 #pragma unroll
         for (int e = 0; e < 4; ++e) ps[4 * ks + e] = pv[e] + pv[e + 4];
-        pb[ks] = u32x4{pack_bf_hw(pv[0], pv[1]), pack_bf_hw(pv[2], pv[3]), pack_bf_hw(pv[4], pv[5]),
-                       pack_bf_hw(pv[6], pv[7])};
+        return u32x4{pack_bf_hw(pv[0], pv[1]), pack_bf_hw(pv[2], pv[3]), pack_bf_hw(pv[4], pv[5]),
+                     pack_bf_hw(pv[6], pv[7])};
+      };
+      u32x4 pb = probabilities(0);
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        if (ks < 3) vread(ks + 1, vr[(ks + 1) & 1]);
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+          const u32x2 lo = vr[ks & 1][dt][0], hi = vr[ks & 1][dt][1];
+          o[dt] = mfma_32x32x16(u32x4{lo.x, lo.y, hi.x, hi.y}, pb, o[dt]);
+        }
+        if (ks < 3) pb = probabilities(ks + 1);
+        __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
       for (int w2 = 8; w2 >= 1; w2 >>= 1)
 #pragma unroll
         for (int e = 0; e < w2; ++e) ps[e] += ps[e + w2];
       l_run += ps[0];
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const bf16_t* vrow = vp_ + (16 * ks + tr_key) * kVD;
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-          const u32x2 lo = lds_read_tr16(vrow + tr_off[dt]);            // keys 16ks + 4h + (0..3)
-          const u32x2 hi = lds_read_tr16(vrow + 8 * kVD + tr_off[dt]);  // keys 16ks + 8 + 4h + (0..3)
-          o[dt] = mfma_32x32x16(u32x4{lo.x, lo.y, hi.x, hi.y}, pb[ks], o[dt]);
-        }
-      }
     }
-    // This wave's prefetches have landed in LDS once its vector memory count drains; the barrier
-    // publishes every wave's, and ends every read of the buffers the next tile prefetches into.
+    // This wave's blocks have landed in LDS once its vector memory count drains; the barrier publishes
+    // every wave's, and ends every read of the buffers the next tile refills.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   };
 
-  f32x16 sa[2], sb[2];
-  dma(k, 0, s_k0, 1);
-  if (tiles > 1) dma(k, 1, s_k1, 1);
-  dma(v, 0, s_v0, 4);
+  dma(kbase, 0, s_k0, 1);
+  dma(vbase, 0, s_v0, 4);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  qk(s_k0, sa);
   for (int t = 0; t < tiles; t += 2) {
     if (t + 2 >= tiles && threadIdx.x == 0) *next = (int)sched_take(ctr);
-    step(t, sa, sb, s_k1, s_v0, s_k0, s_v1);
-    if (t + 1 < tiles) step(t + 1, sb, sa, s_k0, s_v1, s_k1, s_v0);
+    step(t, s_k0, s_v0, s_k1, s_v1);
+    if (t + 1 < tiles) step(t + 1, s_k1, s_v1, s_k0, s_v0);
   }
 
   // Normalise and store: lane (n, h) holds O^T[32dt + 8(e/4) + 4h + e%4][query n].
@@ -335,7 +361,7 @@ __global__ __launch_bounds__(64 * kVWaves, 2) void varlen_attention_kernel(
   group();
   if (threadIdx.x == 0) s_item[0] = (int)sched_take(base + grp * kSchedStride);
   __syncthreads();
-  int i = s_item[0];
+  int i = __builtin_amdgcn_readfirstlane(s_item[0]);
   while (true) {
     if (i >= items) {
       // This group's list is done: take from the next group's.
@@ -345,7 +371,7 @@ __global__ __launch_bounds__(64 * kVWaves, 2) void varlen_attention_kernel(
       ++r;
       if (threadIdx.x == 0) s_item[r & 1] = (int)sched_take(base + grp * kSchedStride);
       __syncthreads();
-      i = s_item[r & 1];
+      i = __builtin_amdgcn_readfirstlane(s_item[r & 1]);
       continue;
     }
     int next = 0;
@@ -355,7 +381,7 @@ __global__ __launch_bounds__(64 * kVWaves, 2) void varlen_attention_kernel(
     ++r;
     if (threadIdx.x == 0) s_item[r & 1] = next;
     __syncthreads();
-    i = s_item[r & 1];
+    i = __builtin_amdgcn_readfirstlane(s_item[r & 1]);
   }
   // Every workgroup of the launch has taken its last number once all have counted themselves out.
   if (threadIdx.x == 0 && sched_take(base + 8 * kSchedStride) == (uint32_t)(total - 1)) {
