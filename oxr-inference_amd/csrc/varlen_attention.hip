@@ -51,6 +51,7 @@ constexpr int kVWaves = 4;             // waves per workgroup
 constexpr int kVRows = 32 * kVWaves;   // query rows per workgroup (all q heads of the kv head)
 constexpr int kKeyTile = 64;           // keys per LDS stage
 constexpr int kLoadsPerWave = kKeyTile * kVD * 2 / 1024 / kVWaves;  // 1 KiB direct-to-LDS loads per wave and tensor
+constexpr float kSlack = 8.f;          // log2 of how far a row's maximum may pass its reference (causal kernel)
 constexpr int kPersistentSlots = 64;   // persistent causal launch: workgroups per XCD (two per CU)
 
 // Work counters of the persistent causal launch, per launch slot (the host cycles through
@@ -163,19 +164,33 @@ __device__ __forceinline__ void varlen_item(const bf16_t* __restrict__ q, const 
   const int64_t row_bytes = (int64_t)KV * kVD * 2;
   const char* const kbase = (const char*)(k + ((int64_t)start * KV + kvh) * kVD);
   const char* const vbase = (const char*)(v + ((int64_t)start * KV + kvh) * kVD);
-  auto dma = [&](const char* base, int t, const bf16_t* dst, int rot) __attribute__((always_inline)) {
-    const char* const tile = base + t * kKeyTile * row_bytes;
-    const int last = len - 1 - t * kKeyTile;  // the sequence's last key, in the tile
+  // Lane offsets of a whole tile: block u of the wave is 4 rows further (a scalar), its K rotation 4 chunks.
+  const int row0 = 4 * kLoadsPerWave * wave + (lane >> 4), pos = lane & 15;
+  const uint32_t row_off = (uint32_t)row0 * (uint32_t)row_bytes;
+  uint32_t k_off[kLoadsPerWave];
 #pragma unroll
-    for (int u = 0; u < kLoadsPerWave; ++u) {
-      const int j = kLoadsPerWave * wave + u;  // 1 KiB block: rows 4j .. 4j + 3
-      const int row = 4 * j + (lane >> 4), pos = lane & 15;
-      const uint32_t off = (uint32_t)min(row, last) * (uint32_t)row_bytes + 16 * ((pos - rot * row) & 15);
-      dma_block(tile, off, lds_address(dst) + 1024 * j);
+  for (int u = 0; u < kLoadsPerWave; ++u) k_off[u] = row_off + 16 * ((pos - row0 - 4 * u) & 15);
+  const uint32_t v_off = row_off + 16 * ((pos - 4 * row0) & 15);
+  auto dma = [&](bool is_k, int t, const bf16_t* dst) __attribute__((always_inline)) {
+    const char* const tile = (is_k ? kbase : vbase) + t * kKeyTile * row_bytes;
+    const uint32_t at = lds_address(dst) + 1024 * kLoadsPerWave * wave;
+    const int last = len - 1 - t * kKeyTile;  // the sequence's last key, in the tile
+    if (last >= kKeyTile - 1) {
+#pragma unroll
+      for (int u = 0; u < kLoadsPerWave; ++u)
+        dma_block(tile + 4 * u * row_bytes, is_k ? k_off[u] : v_off, at + 1024 * u);
+    } else {
+#pragma unroll
+      for (int u = 0; u < kLoadsPerWave; ++u) {
+        const int row = row0 + 4 * u;
+        dma_block(tile, (uint32_t)min(row, last) * (uint32_t)row_bytes + 16 * ((pos - (is_k ? row : 4 * row)) & 15),
+                  at + 1024 * u);
+      }
     }
   };
 
-  float m_run = -INFINITY, mc_run = 0.f, l_run = 0.f;
+  float mc_run = 0.f, l_run = 0.f;  // reference maximum times scale_log2, sum of the probabilities
+  bool started = false;            // some key of the row was visible
   f32x16 o[4];
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt)
@@ -201,8 +216,8 @@ __device__ __forceinline__ void varlen_item(const bf16_t* __restrict__ q, const 
   auto step = [&](int t, const bf16_t* kb_, const bf16_t* vb, const bf16_t* kd, const bf16_t* vd)
                   __attribute__((always_inline)) {
     if (t + 1 < tiles) {
-      dma(kbase, t + 1, kd, 1);
-      dma(vbase, t + 1, vd, 4);
+      dma(true, t + 1, kd);
+      dma(false, t + 1, vd);
     }
     const int kt0 = t * kKeyTile;
     if (kt0 <= wave_last) {  // wave-uniform: otherwise every key of this and later tiles is masked
@@ -250,17 +265,18 @@ __device__ __forceinline__ void varlen_item(const bf16_t* __restrict__ q, const 
       }
       // Row maximum (exact in any order) as a tree of three-input maxima (v_max3_f32): 32 scores in
       // 16 instructions instead of 31.
-      const float mx = xor32_max(row_max32(sv));
-      const bool moved = mx > m_run;
+      // The reference maximum moves only when a row's maximum passes it by kSlack: below that the
+      // probabilities are at most 2^kSlack, which costs no precision (bf16 and fp32 keep their relative
+      // rounding, and the sum is divided out), and with 32 rows per wave most tiles raise some row's maximum.
+      const float raw = xor32_max(row_max32(sv)), mx = raw * scale_log2;
+      const bool moved = raw != -INFINITY && (!started || mx > mc_run + kSlack);
       if (__builtin_amdgcn_ballot_w64(moved)) {
-        const float m_new = moved ? mx : m_run;
-        const float mc_new = m_new == -INFINITY ? 0.f : m_new * scale_log2;
-        const float alpha = !moved ? 1.0f : (m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mc_run - mc_new));
+        const float alpha = !moved ? 1.0f : (started ? __builtin_amdgcn_exp2f(mc_run - mx) : 0.f);
         l_run *= alpha;
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
-        m_run = m_new;
-        mc_run = mc_new;
+        mc_run = moved ? mx : mc_run;
+        started |= moved;
       }
       // P^T for key step ks: accumulators 8 (ks % 2) .. +7 of key block ks / 2, in k-slot order.
       // The tile's probabilities are summed as a tree, then added to the running sum.
@@ -299,8 +315,8 @@ __device__ __forceinline__ void varlen_item(const bf16_t* __restrict__ q, const 
     __syncthreads();
   };
 
-  dma(kbase, 0, s_k0, 1);
-  dma(vbase, 0, s_v0, 4);
+  dma(true, 0, s_k0);
+  dma(false, 0, s_v0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   for (int t = 0; t < tiles; t += 2) {
