@@ -51,7 +51,7 @@ constexpr int kVWaves = 4;             // waves per workgroup
 constexpr int kVRows = 32 * kVWaves;   // query rows per workgroup (all q heads of the kv head)
 constexpr int kKeyTile = 64;           // keys per LDS stage
 constexpr int kLoadsPerWave = kKeyTile * kVD * 2 / 1024 / kVWaves;  // 1 KiB direct-to-LDS loads per wave and tensor
-constexpr float kSlack = 8.f;          // log2 of how far a row's maximum may pass its reference (causal kernel)
+constexpr float kSlack = 8.f;          // log2 of how far a row's maximum may pass its reference
 constexpr int kPersistentSlots = 64;   // persistent causal launch: workgroups per XCD (two per CU)
 
 // Work counters of the persistent causal launch, per launch slot (the host cycles through
@@ -466,22 +466,36 @@ __global__ __launch_bounds__(64 * kPWaves, 1) void varlen_attention_pp_kernel(
   const int key_end = kCausal ? min(len, q0 + rph) : len;
   const int tiles = (key_end + kKeyTile - 1) / kKeyTile;
 
-  // Direct-to-LDS tile loads, rotated rows as in varlen_attention_kernel; kPLoadsPerWave 1 KiB
-  // blocks per wave and tensor.
-  auto dma = [&](const bf16_t* src, int t, bf16_t* dst, int rot) __attribute__((always_inline)) {
+  // Tile loads and their lane offsets as in varlen_item, kPLoadsPerWave 1 KiB blocks per wave and tensor.
+  const int64_t row_bytes = (int64_t)KV * kVD * 2;
+  const char* const kbase = (const char*)(k + ((int64_t)start * KV + kvh) * kVD);
+  const char* const vbase = (const char*)(v + ((int64_t)start * KV + kvh) * kVD);
+  const int row0 = 4 * kPLoadsPerWave * wave + (lane >> 4), pos = lane & 15;
+  const uint32_t row_off = (uint32_t)row0 * (uint32_t)row_bytes;
+  uint32_t k_off[kPLoadsPerWave];
 #pragma unroll
-    for (int u = 0; u < kPLoadsPerWave; ++u) {
-      const int j = kPLoadsPerWave * wave + u;
-      const int row = 4 * j + (lane >> 4), pos = lane & 15;
-      const int key = min(t * kKeyTile + row, len - 1);
-      const int64_t base = ((int64_t)(start + key) * KV + kvh) * kVD;
-      __builtin_amdgcn_global_load_lds(
-          (const void __attribute__((address_space(1)))*)(src + base + 8 * ((pos - rot * row) & 15)),
-          (void __attribute__((address_space(3)))*)(dst + 512 * j), 16, 0, 0);
+  for (int u = 0; u < kPLoadsPerWave; ++u) k_off[u] = row_off + 16 * ((pos - row0 - 4 * u) & 15);
+  const uint32_t v_off = row_off + 16 * ((pos - 4 * row0) & 15);
+  auto dma = [&](bool is_k, int t, const bf16_t* dst) __attribute__((always_inline)) {
+    const char* const tile = (is_k ? kbase : vbase) + t * kKeyTile * row_bytes;
+    const uint32_t at = lds_address(dst) + 1024 * kPLoadsPerWave * wave;
+    const int last = len - 1 - t * kKeyTile;  // the sequence's last key, in the tile
+    if (last >= kKeyTile - 1) {
+#pragma unroll
+      for (int u = 0; u < kPLoadsPerWave; ++u)
+        dma_block(tile + 4 * u * row_bytes, is_k ? k_off[u] : v_off, at + 1024 * u);
+    } else {
+#pragma unroll
+      for (int u = 0; u < kPLoadsPerWave; ++u) {
+        const int row = row0 + 4 * u;
+        dma_block(tile, (uint32_t)min(row, last) * (uint32_t)row_bytes + 16 * ((pos - (is_k ? row : 4 * row)) & 15),
+                  at + 1024 * u);
+      }
     }
   };
 
-  float m_run = -INFINITY, mc_run = 0.f, l_run = 0.f;
+  float mc_run = 0.f, l_run = 0.f;  // as in varlen_item
+  bool started = false;
   f32x16 o[4];
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt)
@@ -568,17 +582,15 @@ __global__ __launch_bounds__(64 * kPWaves, 1) void varlen_attention_pp_kernel(
           if (c >= lim_len || (kCausal && c > lim_q)) sv[kb][e] = -INFINITY;
         }
     }
-    const float mx = xor32_max(row_max32(sv));
-    const bool moved = mx > m_run;
+    const float raw = xor32_max(row_max32(sv)), mx = raw * scale_log2;
+    const bool moved = raw != -INFINITY && (!started || mx > mc_run + kSlack);  // as in varlen_item
     if (__builtin_amdgcn_ballot_w64(moved)) {
-      const float m_new = moved ? mx : m_run;
-      const float mc_new = m_new == -INFINITY ? 0.f : m_new * scale_log2;
-      const float alpha = !moved ? 1.0f : (m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mc_run - mc_new));
+      const float alpha = !moved ? 1.0f : (started ? __builtin_amdgcn_exp2f(mc_run - mx) : 0.f);
       l_run *= alpha;
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
-      m_run = m_new;
-      mc_run = mc_new;
+      mc_run = moved ? mx : mc_run;
+      started |= moved;
     }
     float ps[16];
 #pragma unroll
@@ -610,8 +622,8 @@ __global__ __launch_bounds__(64 * kPWaves, 1) void varlen_attention_pp_kernel(
   // its own order), so the register allocator sees one straight sequence per group; both loops pass
   // the same barriers, two per tile.
   auto loads = [&](int t, bf16_t* kd, bf16_t* vd) __attribute__((always_inline)) {
-    if (t + 1 < tiles) dma(v, t + 1, vd, 4);
-    if (t + 2 < tiles) dma(k, t + 2, kd, 1);
+    if (t + 1 < tiles) dma(false, t + 1, vd);
+    if (t + 2 < tiles) dma(true, t + 2, kd);
   };
   auto iteration_a = [&](int t, const bf16_t* kb, const bf16_t* vb, bf16_t* kd, bf16_t* vd)
                          __attribute__((always_inline)) {
@@ -632,10 +644,10 @@ __global__ __launch_bounds__(64 * kPWaves, 1) void varlen_attention_pp_kernel(
 
   // Prologue: K(0) in; phase -1 (A: QK(0); V(0) and K(1) start loading); phase 0 (A: softmax(0);
   // B: QK(0)).
-  dma(k, 0, s_k0, 1);
+  dma(true, 0, s_k0);
   phase_end(true);
-  if (0 < tiles) dma(v, 0, s_v0, 4);
-  if (1 < tiles) dma(k, 1, s_k1, 1);
+  if (0 < tiles) dma(false, 0, s_v0);
+  if (1 < tiles) dma(true, 1, s_k1);
   if (group_a) {
     matrix_phase(-1, s_k0, s_v0);  // QK(0) only
     phase_end(false);
