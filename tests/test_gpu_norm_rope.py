@@ -133,3 +133,38 @@ def test_out_of_range_slot_is_not_written() -> None:
     keep = [i for i in range(8) if i != 1]
     assert bool((flat[keep] == 9.0).all()) and bool((vc.view(-1, KV, D)[keep] == 9.0).all())
 
+
+
+@pytest.mark.parametrize("H,KV", [(1, 1), (2, 1), (8, 4), (9, 4), (20, 3), (32, 8)])
+def test_heads_per_workgroup_edges(H: int, KV: int) -> None:
+    """Head counts below, at and past the 16 heads of a workgroup; waves that mix q, k and v heads."""
+    rng = np.random.default_rng(27)
+    slots = rng.permutation(64)[:5].astype(np.int64)
+    announce("heads", H, KV)
+    _run_case(5, H, KV, 4, 16, seed=28, need_kv=True, slots=slots, positions=rng.integers(0, 500, size=5))
+
+
+def test_non_finite_rows_bit_exact() -> None:
+    """NaN (any payload) and infinities give the canonical NaN where the reference rounds them; V is copied."""
+    rng = np.random.default_rng(29)
+    n, H, KV, D = 4, 3, 2, 128
+    qkv = rng.standard_normal((n, H + 2 * KV, D)).astype(np.float32)
+    x = _bits(torch.from_numpy(qkv).to(torch.bfloat16))
+    x[0, :, 5] = 0xFFC1   # NaN with a payload: the whole row
+    x[1, :, 70] = 0x7F80  # infinity: NaN at that element and its pair, zeros elsewhere
+    x[2] = 0
+    x[3, 1, :] = 0x7F7F   # the largest finite value: the sum of squares overflows
+    w = _bits(torch.from_numpy(rng.uniform(0.5, 1.5, D).astype(np.float32)).to(torch.bfloat16))
+    cos, sin = norm_rope.rope_tables(n)
+    kc = torch.zeros(1, 16, KV, D, dtype=torch.bfloat16, device="cuda")
+    vc = torch.zeros_like(kc)
+    slots = np.arange(n)
+    announce("non-finite")
+    q, k, v = kernels.qk_norm_rope_store(_dev(x.reshape(n, -1)), _dev(w), _dev(w), _dev(cos), _dev(sin), 1e-6, kc, vc,
+                                         torch.from_numpy(slots).cuda(), H, KV, D, need_kv=True)
+    torch.cuda.synchronize()
+    with np.errstate(all="ignore"):
+        wq, wk, wv = norm_rope.qk_norm_rope_store(x.reshape(n, -1), w, w, cos, sin, 1e-6,
+                                                  np.zeros((n, 1, KV, D), np.uint16), np.zeros((n, 1, KV, D), np.uint16),
+                                                  slots, H, KV, D, need_kv=True)
+    assert np.array_equal(_bits(q), wq) and np.array_equal(_bits(k), wk) and np.array_equal(_bits(v), wv)
