@@ -44,7 +44,7 @@ struct KernelArgs {
 // (s_nop: the wait state between writing m0 and its use.)
 __device__ __forceinline__ void dma_block(const char* base, uint32_t offset, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base)
-               : "memory", "m0");
+               : "memory");
 }
 
 template <int N>

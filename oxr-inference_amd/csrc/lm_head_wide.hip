@@ -49,11 +49,11 @@ __device__ __forceinline__ f32x16 mfma_32x32x16(const u32x4& a, const u32x4& b, 
 // One 1 KiB block from memory into LDS, invisible to the compiler's counters (see csrc/gemm_tile.hip).
 __device__ __forceinline__ void dma_block(const char* base, uint32_t offset, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base)
-               : "memory", "m0");
+               : "memory");
 }
 __device__ __forceinline__ void dma_block_nt(const char* base, uint32_t offset, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(offset), "s"(base)
-               : "memory", "m0");
+               : "memory");
 }
 
 template <int N>

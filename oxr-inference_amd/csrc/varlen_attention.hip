@@ -79,7 +79,7 @@ __device__ __forceinline__ f32x16 mfma_32x32x16(const u32x4& a, const u32x4& b, 
 // and barriers of the tile loop order them.  (s_nop: wait states between the scalar writes and their use.)
 __device__ __forceinline__ void dma_block(const char* base, uint32_t offset, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base)
-               : "memory", "m0");
+               : "memory");
 }
 __device__ __forceinline__ uint32_t lds_address(const bf16_t* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) bf16_t*)p;
