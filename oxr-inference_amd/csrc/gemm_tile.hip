@@ -14,10 +14,10 @@
 // * Within a stage fragments are read two products ahead, with a scheduling barrier per step: left alone
 //   the compiler reads each fragment right before its use and waits for the LDS latency 16 times a stage
 //   (256 x 256 tile, K = 2048, 4096 x 4096: 65 us; read ahead 56).
-// What bounds it: LDS bandwidth (128 bytes a clock).  A stage of the 256 x 256 tile is 2048 matrix core
-// cycles and 192 KB of fragment reads + 64 KB of arriving blocks = 2048 LDS cycles; smaller tiles read more
-// per product.  4 waves of 128 x 128 read less (1536 cycles) but leave one wave per SIMD, whose waits
-// nothing covers: 71 us against 56.
+// What bounds it.  Large tiles (4096 rows): the matrix cores are busy 62% of the CU cycles (256 x 256) and 58%
+// (256 x 128), LDS reads 23 to 29%; the rest is stage barriers and waits that two waves per SIMD do not cover.
+// 4 waves of 128 x 128 read a quarter less LDS but leave one wave per SIMD: 71 us against 56.  Small tiles (up to
+// 256 rows): matrix cores 33%, LDS 24%; the chain of stages waits on memory (see kPer below).
 #include <algorithm>
 
 #include "gemm_tile.h"
@@ -207,7 +207,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(1,
     const bool more = c + STAGES - 1 < stages;
     const int fill = buf == 0 ? STAGES - 1 : buf - 1;
     // Steps of one 16-token piece times the wave's weight pieces; fragments are read two steps ahead, the
-    // next k32 step's weight fragments during this one's steps, the next stage's blocks one per step.
+    // next k32 step's weight fragments during this one's steps.
     constexpr int kSteps = kTM * 2 * kSub;
     const char* at = lds + buf * kStageBytes;
     u32x4 xv[kSteps], wv[2 * kSub][kTN];
@@ -223,7 +223,10 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(1,
     read_x(0);
     read_x(1);
     __builtin_amdgcn_sched_barrier(0);
-    constexpr int kPer = (kL + kSteps - 1) / kSteps;
+    // The next stage's blocks: one a step for the large tiles, all in the first step for the others, whose chain
+    // of stages waits on memory (one 128 x 128 tile alone takes as long as a launch of 192): MLP at 256 rows
+    // 46.4-46.9 us one a step, 45.7-46.0 at once; a prompt's projections on the large tiles 367.7-368.4 / 369.
+    constexpr int kPer = kParts ? kL : (kL + kSteps - 1) / kSteps;
 #pragma unroll
     for (int q = 0; q < kSteps; ++q) {
       if (q + 2 < kSteps) read_x(q + 2);
