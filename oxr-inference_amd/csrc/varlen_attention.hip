@@ -40,6 +40,7 @@
 #include <atomic>
 
 #include "common.h"
+#include "query_tiles.h"
 
 namespace oxr {
 namespace {
@@ -265,7 +266,7 @@ __device__ __forceinline__ void varlen_item(const bf16_t* __restrict__ q, const 
       // 16 instructions instead of 31.
       // Every raise of a row's maximum rescales, so that the largest probability is exactly 1: left unrescaled up to
       // 2^8 it rounds to bf16 like the others, and the error against 64 bits grows (8 x 4096 tokens 1.99e-3 to
-      // 2.05e-3, six sequences of 1023 to 1914 tokens bidirectional 2.24e-3 to 2.33e-3) for 3% of the time.
+      // 2.05e-3, six sequences of 1023 to 1914 tokens bidirectional 2.24e-3 to 2.33e-3) for 6% of the time.
       const float mx = xor32_max(row_max32(sv));
       const bool moved = mx > m_run;
       if (__builtin_amdgcn_ballot_w64(moved)) {
@@ -422,24 +423,18 @@ constexpr int kPLoadsPerWave = kKeyTile * kVD * 2 / 1024 / kPWaves;
 template <bool kCausal>
 __global__ __launch_bounds__(64 * kPWaves, 1) void varlen_attention_pp_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
-    const int32_t* __restrict__ cu_seqlens, int H, int KV, int num_qtiles, int parts, float scale_log2,
-    bf16_t* __restrict__ out) {
+    const int32_t* __restrict__ cu_seqlens, int H, int KV, int num_qtiles, int num_pairs, int log2_parts,
+    float scale_log2, bf16_t* __restrict__ out) {
   __shared__ bf16_t s_k0[kKeyTile * kVD], s_k1[kKeyTile * kVD];
   __shared__ bf16_t s_v0[kKeyTile * kVD], s_v1[kKeyTile * kVD];
 
-  // Units -- a pair, or with KV no multiple of 8 one of the `parts` interleaved parts of its query tiles -- are
-  // dealt to the XCDs in turn (workgroup b runs on XCD b % 8), each XCD taking its units one after another.
-  // So a unit's K/V stays in one L2 and every XCD gets the same share of every sequence.  A contiguous eighth
-  // of the items per XCD gave the XCDs unequal lengths: 6 sequences of 1023 to 1914 tokens (16/8 heads) took
-  // 185 us that way, 158 this way.  (Longest sequence first: 161.)
-  const int per_unit = (num_qtiles + parts - 1) / parts, slot = (int)blockIdx.x >> 3;
-  const int unit = ((int)blockIdx.x & 7) + 8 * (slot / per_unit);
-  const int pair = unit / parts, qt = num_qtiles - 1 - (unit % parts + parts * (slot % per_unit));
-  if (qt < 0) return;  // whole workgroup: before any barrier
+  const QueryTile item = query_tile((int)blockIdx.x, num_qtiles, log2_parts);
+  const int pair = item.pair;
+  if (pair >= num_pairs) return;  // whole workgroup: before any barrier
   const int seq = pair / KV, kvh = pair - seq * KV;
   const int start = cu_seqlens[seq], len = cu_seqlens[seq + 1] - start;
   const int G = H / KV, rph = kPRows / G;
-  const int q0 = qt * rph;
+  const int q0 = item.tile * rph;
   if (q0 >= len) return;  // whole workgroup: before any barrier
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -710,10 +705,10 @@ extern "C" int oxr_varlen_attention(const oxr_bf16* q, const oxr_bf16* k, const 
   hipStream_t s = (hipStream_t)stream;
   const int num_pairs = num_seqs * num_kv_heads;
   if (!causal) {
-    const int parts = num_kv_heads % 8 == 0 ? 1 : num_kv_heads % 4 == 0 ? 2 : num_kv_heads % 2 == 0 ? 4 : 8;
-    const dim3 grid((unsigned)num_pairs * parts * ((num_qtiles + parts - 1) / parts));
+    const int parts = log2_parts(num_kv_heads, num_pairs, num_qtiles);
+    const dim3 grid((unsigned)query_tile_blocks(num_pairs, num_qtiles, parts));
     hipLaunchKernelGGL(varlen_attention_pp_kernel<false>, grid, dim3(64 * kPWaves), 0, s, q, k, v, cu_seqlens,
-                       num_heads, num_kv_heads, num_qtiles, parts, scale_log2, out);
+                       num_heads, num_kv_heads, num_qtiles, num_pairs, parts, scale_log2, out);
   } else {
     // Two workgroups per CU, or fewer when the largest XCD group has fewer items.
     static std::atomic<uint32_t> launches{0};
