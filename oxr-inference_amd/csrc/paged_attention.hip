@@ -171,62 +171,6 @@ struct RopeArgs {
   bf16_t* v_store;
 };
 
-// kStream launches: every context counted in 32-key units (at least one), the batch's units end to end, share
-// j of n the units [begin(j), begin(j + 1)).  A share's partials go to unit 2j for a piece at its start and
-// 2j + 1 for one that begins inside it and goes on in the next share.  When the shares would not shorten the
-// longest context by more than 16 units (512 keys: a piece costs about that much besides its keys), `whole`
-// gives every workgroup one context.
-constexpr int kStreamMaxBatch = 256;
-struct StreamSplit {
-  int prefix[kStreamMaxBatch + 1];  // units before each context
-  int len[kStreamMaxBatch];
-  int wave_units[kWaves], wave_longest[kWaves];
-  int total, longest;
-  bool whole;
-  __device__ __forceinline__ int begin(int j, int n) const { return (int)((int64_t)j * total / n); }
-};
-
-// Fills `sp` (LDS) with THREADS >= batch threads; every thread of the workgroup takes part.
-template <int THREADS>
-__device__ __forceinline__ void stream_split(StreamSplit& sp, const int32_t* __restrict__ seq_lens, int batch,
-                                             int max_seq_len, int n) {
-  static_assert(THREADS >= kStreamMaxBatch && THREADS % kWave == 0, "one context per thread");
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int len = t < batch ? max(0, min(seq_lens[t], max_seq_len)) : 0;
-  const int units = t < batch ? max(1, (len + 31) / 32) : 0;
-  int sum = units, longest = units;
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const int up = __shfl_up(sum, d, kWave);
-    if (lane >= d) sum += up;
-    longest = max(longest, __shfl_xor(longest, d, kWave));
-  }
-  if (lane == 63) {
-    sp.wave_units[wave] = sum;
-    sp.wave_longest[wave] = longest;
-  }
-  __syncthreads();
-  int before = 0, total = 0;
-  longest = 0;
-#pragma unroll
-  for (int w = 0; w < THREADS / kWave; ++w) {
-    if (w < wave) before += sp.wave_units[w];
-    total += sp.wave_units[w];
-    longest = max(longest, sp.wave_longest[w]);
-  }
-  if (t < batch) {
-    sp.prefix[t + 1] = before + sum;
-    sp.len[t] = len;
-  }
-  if (t == 0) {
-    sp.prefix[0] = 0;
-    sp.total = total;
-    sp.longest = longest;
-    sp.whole = longest <= (total + n - 1) / n + 16;
-  }
-  __syncthreads();
-}
-
 // kFused: q comes from qkv through norm + RoPE (done here, into LDS), and the
 // new tokens' K (norm + RoPE) and V rows are written to the cache by the
 // workgroup whose key range holds their positions, before any wave reads them;
@@ -236,16 +180,12 @@ __device__ __forceinline__ void stream_split(StreamSplit& sp, const int32_t* __r
 // is multiplied by each tile, and the V^T fragments are shared by the tiles.
 // JR: rounds of the fused prologue's 32 row jobs (HPW * (R + 2 S) <= 32 * JR).
 // kPlanned: pieces from a plan (paged_extend_plan_kernel); otherwise `splits` even pieces per context.
-// kStream: the batch's contexts end to end, cut into `splits` equal shares of 32-key units (StreamSplit);
-// workgroup (head group, share) takes the pieces of contexts in its share one after another.  (Head groups
-// are neighbours in dispatch order: they read neighbouring slices of the same token rows.)
-template <bool kFused, int HPW, int NT, int JR, bool kPlanned, bool kStream = false>
+template <bool kFused, int HPW, int NT, int JR, bool kPlanned>
 __global__ __launch_bounds__(64 * kWaves) void paged_extend_kernel(
     const bf16_t* __restrict__ q, const bf16_t* k_cache, const bf16_t* v_cache, const int32_t* __restrict__ seq_lens,
     const int32_t* __restrict__ block_table, int64_t table_stride, int S, int H, int KV, int log2_bs,
     int64_t num_blocks, float scale_log2, int max_seq_len, int splits, const int32_t* __restrict__ plan,
-    float* __restrict__ part_o, float* __restrict__ part_ml, bf16_t* __restrict__ out, int out_packed, RopeArgs ra,
-    int batch) {
+    float* __restrict__ part_o, float* __restrict__ part_ml, bf16_t* __restrict__ out, int out_packed, RopeArgs ra) {
   constexpr int kStreams = kWaves / HPW;  // waves per kv head
   // Two row tiles' q fragments (32 registers) would not fit next to two tiles'
   // accumulators and the two pair buffers: with NT = 2 the MFMAs read them from LDS.
@@ -257,22 +197,29 @@ __global__ __launch_bounds__(64 * kWaves) void paged_extend_kernel(
   __shared__ float s_m[kWaves][16], s_l[kWaves][16];
   __shared__ int s_pages[kMaxSpanPages];
 
+  // Which piece of which context this workgroup takes: piece blockIdx.x of sequence blockIdx.z of
+  // `splits` even pieces, or, with a plan (paged_extend_plan_kernel), the entry of its slot.  A plan
+  // whose header names another batch or split count was written for another launch: the launch then
+  // runs on even pieces (the merge makes the same test), which read and write the same units.
+  int split = blockIdx.x, b = blockIdx.z, pieces = 0;
+  const bool use_plan = kPlanned && plan[0] == (int)gridDim.z && plan[1] == splits;
+  if (use_plan) {
+    const int a = plan[kPlanHead + gridDim.z + blockIdx.z * splits + blockIdx.x];
+    // A spare slot the plan leaves idle (workgroup-uniform); entries out of range (a plan written for
+    // another launch) are treated alike, so nothing is addressed outside the launch's arrays.
+    if (a < 0 || (a >> 8) >= (int)gridDim.z || (a & 255) >= 2 * splits) return;
+    b = a >> 8;
+    split = a & 255;
+    pieces = min(max(plan[kPlanHead + b], 1), 2 * splits);
+  }
   const int G = H / KV, R = S * G;
-  const int head_group = kStream ? blockIdx.x : blockIdx.y;  // kv heads [HPW * head_group, +HPW)
-
-  // One piece: keys [stream_begin, stream_end) of sequence b (kStream, partial unit `split`), else piece `split`.
-  auto run_piece = [&](const int b, const int split, const int pieces, const bool use_plan, const int stream_len,
-                       const int stream_begin, const int stream_end) __attribute__((always_inline)) {
-  int tid = threadIdx.x;
-  // (kStream: per-lane values are formed anew for each piece; kept across pieces they would spill.)
-  if constexpr (kStream) asm volatile("" : "+v"(tid));
-  const int lane = tid % kWave;
+  const int tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);  // wave-uniform, so its addressing is scalar
   const int r = lane & 15, g = lane >> 4;
-  // The workgroup owns kv heads [HPW * head_group, +HPW): wave w serves head
+  // The workgroup owns kv heads [HPW * blockIdx.y, +HPW): wave w serves head
   // slot w % HPW and walks that head's keys as stream w / HPW of kStreams.
   const int hs = wave % HPW, stream = wave / HPW;
-  const int kvh = head_group * HPW + hs;
+  const int kvh = (int)blockIdx.y * HPW + hs;
 
   // Fused: HPW * (R + 2S) row jobs of one 128-element row each, on 16 lanes, in
   // JR rounds of 32 -- per head slot, q rows [0, R), then the K rows and the V
@@ -301,7 +248,7 @@ __global__ __launch_bounds__(64 * kWaves) void paged_extend_kernel(
       const int jv = f_valid[jr] ? job : 0;
       f_hs[jr] = jv / f_per_head;
       f_jj[jr] = jv % f_per_head;
-      const int kvh_j = head_group * HPW + f_hs[jr];
+      const int kvh_j = (int)blockIdx.y * HPW + f_hs[jr];
       int head;
       if (f_jj[jr] < R) {
         f_ss[jr] = f_jj[jr] / G;
@@ -321,7 +268,7 @@ __global__ __launch_bounds__(64 * kWaves) void paged_extend_kernel(
     }
   }
 
-  const int L = kStream ? stream_len : min(seq_lens[b], max_seq_len);  // max_seq_len <= table span (host check)
+  const int L = min(seq_lens[b], max_seq_len);  // max_seq_len <= table span, checked on the host
 
   // This workgroup's keys: piece `split` of [0, L), in whole 32-key pairs.
   // (A plan's pieces are never longer than an even split of max_seq_len; the clamp keeps the page
@@ -329,14 +276,13 @@ __global__ __launch_bounds__(64 * kWaves) void paged_extend_kernel(
   const int span = use_plan ? min(((L + pieces - 1) / pieces + 31) / 32 * 32,
                                   ((max_seq_len + splits - 1) / splits + 31) / 32 * 32)
                             : ((L + splits - 1) / splits + 31) / 32 * 32;
-  const int t_begin = kStream ? stream_begin : split * span;
-  const int t_end = kStream ? stream_end : min(L, t_begin + span);
-  // Whether the whole context is in this piece.
-  const bool single = kStream ? t_begin == 0 && t_end == L : use_plan ? pieces == 1 : L <= span;
+  const int t_begin = split * span;
+  const int t_end = min(L, t_begin + span);
+  const bool single = use_plan ? pieces == 1 : L <= span;  // the whole context is in piece 0
   // A plan built from other (shorter) lengths can leave keys past its pieces; that sequence's rows
   // are then written as NaN (here when it has one piece, else by the merge) instead of dropping keys.
   const bool uncovered = use_plan && (int64_t)pieces * span < L;
-  if (!kStream && single && split > 0) return;
+  if (single && split > 0) return;
   const int32_t* table_row = block_table + (int64_t)b * table_stride;
 
   // This split's page numbers (as stored; clamped when read), staged into LDS below.  One entry per thread
@@ -405,7 +351,7 @@ __global__ __launch_bounds__(64 * kWaves) void paged_extend_kernel(
         else s_newv[f_hs[jr]][f_ss[jr]][f_s16] = f_raw[jr];
         const int pos = L - S + f_ss[jr];
         if (pos >= t_begin && pos < t_end && f_slot[jr] >= 0 && f_slot[jr] < ra.num_slots) {
-          const int kvh_j = head_group * HPW + f_hs[jr];
+          const int kvh_j = (int)blockIdx.y * HPW + f_hs[jr];
           bf16_t* dst = (is_k ? ra.k_store : ra.v_store) + (f_slot[jr] * KV + kvh_j) * kD + f_s16 * 8;
           st128(dst, is_k ? normed : f_raw[jr]);
         }
@@ -595,12 +541,10 @@ __global__ __launch_bounds__(64 * kWaves) void paged_extend_kernel(
     for (int idx = tid; idx < HPW * rows * (kD / 4); idx += 64 * kWaves) {
       const int ho = idx / (rows * (kD / 4)), rl = (idx / (kD / 4)) % rows, d0 = (idx % (kD / 4)) * 4;
       const int rr = 16 * t + rl;
-      const int kvh_o = head_group * HPW + ho;
+      const int kvh_o = (int)blockIdx.y * HPW + ho;
       // Even: the (sequence, piece) unit; planned: this workgroup's own slot (the plan maps pieces to slots).
-      const int64_t unit = kStream    ? (int64_t)kvh_o * 2 * splits + split
-                           : use_plan ? ((int64_t)blockIdx.z * KV + kvh_o) * splits + blockIdx.x
-                                      : ((int64_t)b * KV + kvh_o) * splits + split;
-      const int64_t part_row = unit * (kStream ? R : kPartRows) + rr;
+      const int64_t unit = use_plan ? ((int64_t)blockIdx.z * KV + kvh_o) * splits + blockIdx.x
+                                    : ((int64_t)b * KV + kvh_o) * splits + split;
       float mmax = -INFINITY;
 #pragma unroll
       for (int k = 0; k < kStreams; ++k) mmax = fmaxf(mmax, s_m[ho + HPW * k][rl]);
@@ -621,57 +565,11 @@ __global__ __launch_bounds__(64 * kWaves) void paged_extend_kernel(
         dst[0] = pack_bf(acc[0] * inv, acc[1] * inv);
         dst[1] = pack_bf(acc[2] * inv, acc[3] * inv);
       } else {
-        f32x4* const po = reinterpret_cast<f32x4*>(part_o + part_row * kD + d0);
+        f32x4* const po = reinterpret_cast<f32x4*>(part_o + (unit * kPartRows + rr) * kD + d0);
         *po = acc;
-        if (d0 == 0) *reinterpret_cast<f32x2*>(part_ml + part_row * 2) = f32x2{mmax, l};
+        if (d0 == 0) *reinterpret_cast<f32x2*>(part_ml + (unit * kPartRows + rr) * 2) = f32x2{mmax, l};
       }
     }
-  }
-  };
-
-  if constexpr (kStream) {
-    __shared__ StreamSplit sp;
-    stream_split<64 * kWaves>(sp, seq_lens, batch, max_seq_len, splits);
-    const int slot = blockIdx.y;
-    if (sp.whole) {
-      if (slot < batch) run_piece(slot, 0, 0, false, sp.len[slot], 0, sp.len[slot]);
-      return;
-    }
-    if (slot >= splits) return;
-    const int u0 = sp.begin(slot, splits), u1 = sp.begin(slot + 1, splits);
-    // The context that holds unit u0 (a bisection over the prefix sums).
-    int lo = 0, hi = batch;
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (sp.prefix[mid] <= u0) lo = mid;
-      else hi = mid;
-    }
-    for (int c = __builtin_amdgcn_readfirstlane(lo); c < batch; ++c) {
-      const int first = __builtin_amdgcn_readfirstlane(sp.prefix[c]);
-      const int last = __builtin_amdgcn_readfirstlane(sp.prefix[c + 1]);
-      if (first >= u1) break;
-      const int len = __builtin_amdgcn_readfirstlane(sp.len[c]);
-      run_piece(c, 2 * slot + (first <= u0 ? 0 : 1), 0, false, len, 32 * (max(first, u0) - first),
-                min(len, 32 * (min(last, u1) - first)));
-      __syncthreads();  // the next piece refills the LDS arrays
-    }
-  } else {
-    // Which piece of which context this workgroup takes: piece blockIdx.x of sequence blockIdx.z of
-    // `splits` even pieces, or, with a plan (paged_extend_plan_kernel), the entry of its slot.  A plan
-    // whose header names another batch or split count was written for another launch: the launch then
-    // runs on even pieces (the merge makes the same test), which read and write the same units.
-    int split = blockIdx.x, b = blockIdx.z, pieces = 0;
-    const bool use_plan = kPlanned && plan[0] == (int)gridDim.z && plan[1] == splits;
-    if (use_plan) {
-      const int a = plan[kPlanHead + gridDim.z + blockIdx.z * splits + blockIdx.x];
-      // A spare slot the plan leaves idle (workgroup-uniform); entries out of range (a plan written for
-      // another launch) are treated alike, so nothing is addressed outside the launch's arrays.
-      if (a < 0 || (a >> 8) >= (int)gridDim.z || (a & 255) >= 2 * splits) return;
-      b = a >> 8;
-      split = a & 255;
-      pieces = min(max(plan[kPlanHead + b], 1), 2 * splits);
-    }
-    run_piece(b, split, pieces, use_plan, 0, 0, 0);
   }
 }
 
@@ -812,56 +710,6 @@ __global__ __launch_bounds__(kPartRows * kD / 4) void paged_extend_merge_kernel(
   dst[1] = pack_bf(acc[2] * inv, acc[3] * inv);
 }
 
-// The merge of a kStream launch: piece i of a context is in share j + i, j the share of its first unit; a
-// context inside one share was stored by the main kernel.
-constexpr int kStreamMergeThreads = 256;
-__global__ __launch_bounds__(kStreamMergeThreads) void paged_extend_stream_merge_kernel(
-    const float* __restrict__ part_o, const float* __restrict__ part_ml, const int32_t* __restrict__ seq_lens, int S,
-    int H, int KV, int max_seq_len, int n, int batch, bf16_t* __restrict__ out, int out_packed) {
-  constexpr int kChunk = 8;  // pieces whose partials are requested together
-  __shared__ StreamSplit sp;
-  stream_split<kStreamMergeThreads>(sp, seq_lens, batch, max_seq_len, n);
-  if (sp.whole) return;
-  const int b = blockIdx.x, G = H / KV, R = S * G;
-  const int64_t total = sp.total;
-  auto share_of = [&](int64_t unit) { return (int)(((unit + 1) * n - 1) / total); };
-  const int first = sp.prefix[b], j0 = share_of(first), pieces = share_of(sp.prefix[b + 1] - 1) - j0 + 1;
-  if (pieces == 1) return;
-  const int first_unit = 2 * j0 + (first <= sp.begin(j0, n) ? 0 : 1);
-  for (int idx = threadIdx.x; idx < KV * R * (kD / 4); idx += kStreamMergeThreads) {
-    const int kvh = idx / (R * (kD / 4)), rr = idx / (kD / 4) % R, d0 = idx % (kD / 4) * 4;
-    const int64_t unit0 = (int64_t)kvh * 2 * n;
-    float m = -INFINITY, l = 0.f;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int c0 = 0; c0 < pieces; c0 += kChunk) {
-      f32x2 ml[kChunk];
-      f32x4 v[kChunk];
-#pragma unroll
-      for (int j = 0; j < kChunk; ++j) {  // past the last piece: the last, weight 0 below
-        const int i = min(c0 + j, pieces - 1);
-        const int64_t row = (unit0 + (i == 0 ? first_unit : 2 * (j0 + i))) * R + rr;
-        ml[j] = *reinterpret_cast<const f32x2*>(part_ml + row * 2);
-        v[j] = *reinterpret_cast<const f32x4*>(part_o + row * kD + d0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < kChunk; ++j) {
-        const float mj = c0 + j < pieces ? ml[j][0] : -INFINITY;
-        const float mn = fmaxf(m, mj);
-        const float mu = (mn == -INFINITY) ? 0.f : mn;
-        const float a = exp2f(m - mu), w = exp2f(mj - mu);
-        l = l * a + ml[j][1] * w;
-        acc = acc * a + v[j] * w;
-        m = mn;
-      }
-    }
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
-    uint32_t* dst = out_vec(out, (int64_t)b * S + rr / G, (kvh * G + rr % G) * kD + d0, H * kD, out_packed);
-    dst[0] = pack_bf(acc[0] * inv, acc[1] * inv);
-    dst[1] = pack_bf(acc[2] * inv, acc[3] * inv);
-  }
-}
-
 // A plan of context pieces for one launch (oxr_paged_extend_plan), so that contexts of different
 // lengths take workgroups in proportion.  Without one, every context is cut into the launch's
 // `splits` pieces and the longest bounds the launch.  One piece length serves the whole batch:
@@ -990,7 +838,7 @@ namespace {
 // any batch' <= batch (smaller batches split their contexts further, so a workspace sized for a batch
 // serves every smaller one).  A planned launch writes one partial per workgroup slot too.  (A launch
 // with one split stores its output directly and needs none.)
-size_t partial_units(int32_t batch, int32_t num_kv_heads, int32_t max_seq_len) {
+size_t partial_bytes(int32_t batch, int32_t num_kv_heads, int32_t max_seq_len) {
   if (batch <= 0 || num_kv_heads <= 0 || max_seq_len <= 0) return 0;
   size_t units = 0;
   for (int32_t bb = 1; bb <= batch; ++bb)
@@ -999,37 +847,7 @@ size_t partial_units(int32_t batch, int32_t num_kv_heads, int32_t max_seq_len) {
         const int splits = splits_for(bb, num_kv_heads, hpw, max_seq_len);
         if (splits > 1) units = std::max(units, (size_t)bb * num_kv_heads * splits);
       }
-  return units;
-}
-size_t partial_bytes(int32_t batch, int32_t num_kv_heads, int32_t max_seq_len) {
-  return partial_units(batch, num_kv_heads, max_seq_len) * kPartRows * (kD + 2) * sizeof(float);
-}
-
-// A kStream launch: kv heads per workgroup and shares (one workgroup per CU); no shares: a workgroup per context
-// and head group instead.  Streams take over where that would be the launch and would fill the chip less than
-// twice, at 256 to 479 (context, head group) units: there contexts of different lengths leave CUs idle behind
-// the longest (a workgroup streams at most 50 GB/s).  Decode, 16/8 heads, us, without and with: 64 contexts of
-// 256-8192 keys 226 / 199, 96 of 200-3000 165 / 125; 64 of about 2020 keys 89 / 92 (the merge launch finds
-// nothing to do); 128 of 200-3000, 8/8 heads, two rounds of workgroups: 170 / 173.  Two 4-wave workgroups per
-// CU: 203 and 105 for the first and third.  Below 256 units contexts are split evenly or by a plan.  The
-// partials (two units of R rows a share) fit the workspace of the batch.  Contexts of up to 1024 keys are too
-// short to share: 64 of 500-600 keys 30 / 34.
-constexpr int kMinStreamKeys = 1024;
-constexpr int kMaxStreamUnits = 480;
-struct StreamLaunch {
-  int hpw, shares;
-};
-StreamLaunch stream_launch(int32_t batch, int32_t tokens_per_seq, int32_t num_heads, int32_t num_kv_heads,
-                           int32_t max_seq_len, int splits) {
-  const int rows = tokens_per_seq * (num_heads / num_kv_heads);
-  const int jobs = tokens_per_seq * (num_heads / num_kv_heads + 2);  // per head
-  const int hpw = num_kv_heads % 2 == 0 && 2 * jobs <= kJobSlots ? 2 : 1;
-  if (splits != 1 || batch > kStreamMaxBatch || rows > 16 || jobs > kJobSlots || max_seq_len <= kMinStreamKeys ||
-      batch * (num_kv_heads / hpw) >= kMaxStreamUnits)
-    return {1, 0};
-  const int64_t room = (int64_t)partial_units(batch, num_kv_heads, max_seq_len) * kPartRows;
-  const int64_t shares = std::min<int64_t>(256 / (num_kv_heads / hpw), room / (2 * (int64_t)num_kv_heads * rows));
-  return {hpw, shares >= 16 ? (int)shares : 0};
+  return units * kPartRows * (kD + 2) * sizeof(float);
 }
 
 }  // namespace
@@ -1073,32 +891,6 @@ int launch_paged_extend(const oxr_bf16* q, const oxr_bf16* k_cache, const oxr_bf
   int log2_bs = 0;
   while ((1 << log2_bs) < block_size) ++log2_bs;
   float* part_o = static_cast<float*>(workspace);
-  const StreamLaunch st = stream_launch(batch, tokens_per_seq, num_heads, num_kv_heads, max_seq_len, splits);
-  if (st.shares > 0) {
-    const int shares = st.shares;
-    const int rows = tokens_per_seq * (num_heads / num_kv_heads);
-    float* part_ml = part_o + (size_t)num_kv_heads * 2 * shares * rows * kD;
-    const RopeArgs rope = ra ? *ra : RopeArgs{};
-    const float scale_log2 = scale * 1.4426950408889634f;
-    auto launch = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3(num_kv_heads / st.hpw, std::max(shares, (int)batch)), dim3(64 * kWaves), 0, s,
-                         ra ? nullptr : q, k_cache, v_cache, seq_lens, block_table, table_stride, tokens_per_seq,
-                         num_heads, num_kv_heads, log2_bs, num_blocks, scale_log2, max_seq_len, shares, nullptr,
-                         part_o, part_ml, out, out_packed, rope, batch);
-    };
-    if (!ra) {
-      if (st.hpw == 2) launch(paged_extend_kernel<false, 2, 1, 1, false, true>);
-      else launch(paged_extend_kernel<false, 1, 1, 1, false, true>);
-    } else {
-      if (st.hpw == 2) launch(paged_extend_kernel<true, 2, 1, 1, false, true>);
-      else launch(paged_extend_kernel<true, 1, 1, 1, false, true>);
-    }
-    const int status = OXR_LAUNCH_STATUS();
-    if (status) return status;
-    hipLaunchKernelGGL(paged_extend_stream_merge_kernel, dim3(batch), dim3(kStreamMergeThreads), 0, s, part_o, part_ml,
-                       seq_lens, tokens_per_seq, num_heads, num_kv_heads, max_seq_len, shares, batch, out, out_packed);
-    return OXR_LAUNCH_STATUS();
-  }
   if (splits == 1) plan = nullptr;  // nothing to balance: every context is one piece
   float* part_ml = part_o + (size_t)batch * num_kv_heads * splits * kPartRows * kD;
   const float scale_log2 = scale * 1.4426950408889634f;
@@ -1107,9 +899,8 @@ int launch_paged_extend(const oxr_bf16* q, const oxr_bf16* k_cache, const oxr_bf
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, block, 0, s, ra ? nullptr : q, k_cache, v_cache, seq_lens, block_table,
                        table_stride, tokens_per_seq, num_heads, num_kv_heads, log2_bs, num_blocks, scale_log2,
-                       max_seq_len, splits, plan, part_o, part_ml, out, out_packed, rope, batch);
-  };
-  auto launch_k = [&](auto even, auto planned) {
+                       max_seq_len, splits, plan, part_o, part_ml, out, out_packed, rope);
+  };  auto launch_k = [&](auto even, auto planned) {
     if (plan) launch(planned);
     else launch(even);
   };

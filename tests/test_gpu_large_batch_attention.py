@@ -1,9 +1,9 @@
-"""Paged attention of large batches, whose contexts are cut into equal shares of the whole batch's keys
-(256 to 479 (context, kv-head group) units): contexts inside one share, over several, starting exactly on a
-share, empty, of one key, and one far longer than the rest; every head grouping, both page sizes, verify and
-decode widths -- against a float64 softmax over the gathered keys, and the fused launch against the separate
-q/k norm + RoPE + store and attention calls bit for bit.  Tolerance: the outputs' bf16 rounding (2^-9) and the
-bf16 rounding of the probabilities (2^-9 of a convex combination of |v| <= 6).
+"""Paged attention of large batches, where every context is one workgroup's work (256 (context, kv-head group)
+units and more): mixed, equal, rising, falling, empty and one-key contexts, contexts longer than ``max_seq_len``,
+sharp scores; every head grouping, both page sizes, verify and decode widths -- against a float64 softmax over the
+gathered keys, and the fused launch against the separate q/k norm + RoPE + store and attention calls bit for bit.
+A context's result depends on neither its neighbours' lengths nor the workspace.  Tolerance: the outputs' bf16
+rounding (2^-8) and the bf16 rounding of the probabilities (2^-8 of a convex combination of |v|).
 """
 
 from __future__ import annotations
@@ -36,21 +36,31 @@ def _batch(lens: list[int], bs: int, kv: int, g: torch.Generator):
 
 
 def _check(out: torch.Tensor, q: torch.Tensor, kc, vc, table, lens: list[int]) -> None:
+    """Every row of every context; a token before its context's first key (fewer keys than tokens) sees none: zeros."""
     _, s, h, _ = q.shape
     kv, bs = kc.shape[2], kc.shape[1]
     for b, n in enumerate(lens):
-        if n < s:
+        pos = n - s + torch.arange(s, device="cuda")
+        assert bool((out[b, pos < 0] == 0).all()), (b, n)
+        if n == 0:
             continue
         at = torch.arange(n, device="cuda")
         slot = table[b].long()[at // bs] * bs + at % bs
         k, v = (c.view(-1, kv, D)[slot].double().repeat_interleave(h // kv, 1) for c in (kc, vc))
-        scores = (q[b].double()[:, :, None, :] * 1.0).permute(1, 0, 2, 3).squeeze(2) @ k.permute(1, 2, 0).contiguous()
-        scores = scores * D ** -0.5
-        scores.masked_fill_(at[None, :] > (n - s + torch.arange(s, device="cuda"))[:, None], float("-inf"))
-        want = (torch.softmax(scores, -1) @ v.permute(1, 0, 2).contiguous()).permute(1, 0, 2)
-        mass = (torch.softmax(scores, -1) @ v.abs().permute(1, 0, 2).contiguous()).permute(1, 0, 2)
+        scores = q[b].double().permute(1, 0, 2).contiguous() @ k.permute(1, 2, 0).contiguous() * D ** -0.5
+        scores.masked_fill_(at[None, :] > pos[:, None], float("-inf"))
+        p = torch.softmax(scores, -1).nan_to_num(0.0)
+        want = (p @ v.permute(1, 0, 2).contiguous()).permute(1, 0, 2)
+        mass = (p @ v.abs().permute(1, 0, 2).contiguous()).permute(1, 0, 2)
         err = (out[b].double() - want).abs()
         assert bool((err <= 2.0 ** -8 * want.abs() + 2.0 ** -8 * mass + 1e-5).all()), (b, n, err.max().item())
+
+
+def _extend(q: torch.Tensor, kc, vc, lens_t, table, **kw) -> torch.Tensor:
+    out = torch.full_like(q, float("nan"))
+    attention.paged_extend(q, kc, vc, lens_t, table, out=out, **kw)
+    torch.cuda.synchronize()
+    return out
 
 
 def _sequences(s: int, h: int, kv: int) -> int:
@@ -69,27 +79,54 @@ def test_mixed_contexts(s: int, h: int, kv: int, bs: int) -> None:
     lens = (MIXED * 4)[: _sequences(s, h, kv)]
     kc, vc, table, lens_t = _batch(lens, bs, kv, g)
     q = torch.randn(len(lens), s, h, D, generator=g, device="cuda").to(torch.bfloat16)
-    announce("stream attention", s, h, kv, bs, len(lens))
-    out = attention.paged_extend(q, kc, vc, lens_t, table)
-    torch.cuda.synchronize()
-    _check(out, q, kc, vc, table, lens)
+    announce("large batch", s, h, kv, bs, len(lens))
+    _check(_extend(q, kc, vc, lens_t, table), q, kc, vc, table, lens)
 
 
-@pytest.mark.parametrize("lens", [[1024] * 64, [1056] * 100, [16] * 63 + [8000], [600] * 110 + [1100], [1025] * 60 + [1] * 59])
+@pytest.mark.parametrize("lens", [[1024] * 64, [1056] * 100, [16] * 63 + [8000], [600] * 110 + [1100], [1025] * 60 + [1] * 59,
+                                  list(range(0, 2600, 40)), list(range(5080, 0, -40)), [33] * 129, [0] * 70,
+                                  [7, 0, 3000, 64] * 48 + [65], [5] * 256 + [300]], ids=lambda l: f"{len(l)}x{l[0]}-{l[-1]}")
 def test_equal_long_and_short_contexts(lens: list[int]) -> None:
-    """Shares that end exactly between contexts, one context that fills many shares, more contexts than shares."""
+    """One round of workgroups and several; lengths alike, one far longer, rising, falling, empty."""
     g = torch.Generator(device="cuda").manual_seed(len(lens))
     kc, vc, table, lens_t = _batch(lens, 16, 8, g)
     q = torch.randn(len(lens), 1, 16, D, generator=g, device="cuda").to(torch.bfloat16)
-    announce("stream lengths", lens[0], lens[-1], len(lens))
-    out = attention.paged_extend(q, kc, vc, lens_t, table)
-    torch.cuda.synchronize()
-    _check(out, q, kc, vc, table, lens)
+    announce("large batch lengths", lens[0], lens[-1], len(lens))
+    _check(_extend(q, kc, vc, lens_t, table), q, kc, vc, table, lens)
+
+
+@pytest.mark.parametrize("s", [1, 4])
+def test_sharp_scores_and_clamped_contexts(s: int) -> None:
+    g = torch.Generator(device="cuda").manual_seed(90 + s)
+    lens = (MIXED * 2)[:70]
+    kc, vc, table, lens_t = _batch(lens, 16, 8, g)
+    q = (12 * torch.randn(len(lens), s, 16, D, generator=g, device="cuda")).to(torch.bfloat16)
+    announce("large batch sharp", s)
+    _check(_extend(q, kc, vc, lens_t, table), q, kc, vc, table, lens)
+    _check(_extend(q, kc, vc, lens_t, table, max_seq_len=1000), q, kc, vc, table, [min(n, 1000) for n in lens])
+
+
+@pytest.mark.parametrize("batch", [64, 96])
+def test_a_context_does_not_depend_on_its_neighbours(batch: int) -> None:
+    """Bit for bit, and nothing is written to the workspace."""
+    g = torch.Generator(device="cuda").manual_seed(batch)
+    lens = (MIXED * 2)[:batch]
+    kc, vc, table, lens_t = _batch([4096] * batch, 256, 8, g)
+    q = torch.randn(batch, 1, 16, D, generator=g, device="cuda").to(torch.bfloat16)
+    workspace = torch.full((attention.workspace_bytes(batch, 8, 4096),), 0xAB, dtype=torch.uint8, device="cuda")
+    lens_t = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    announce("large batch neighbours", batch)
+    full = _extend(q, kc, vc, lens_t, table, workspace=workspace)
+    other = lens_t.clone()
+    other[10:] = other[10:].flip(0) // 3 + 1
+    got = _extend(q, kc, vc, other, table, workspace=workspace)
+    assert torch.equal(got[:10].view(torch.int16), full[:10].view(torch.int16))
+    assert bool((workspace == 0xAB).all())
 
 
 @pytest.mark.parametrize("s,h,kv", [(1, 16, 8), (4, 16, 8), (8, 16, 8), (3, 8, 8)])
 def test_fused_equals_separate_calls(s: int, h: int, kv: int) -> None:
-    """Contexts of at least s keys whose new tokens straddle shares; output and both caches."""
+    """Contexts of at least s keys; output and both caches."""
     g = torch.Generator(device="cuda").manual_seed(s)
     lens = [max(n, s) for n in (MIXED * 4)[: _sequences(s, h, kv)]]
     kc, vc, table, lens_t = _batch(lens, 16, kv, g)
@@ -101,7 +138,7 @@ def test_fused_equals_separate_calls(s: int, h: int, kv: int) -> None:
     pos = (lens_t.long()[:, None] - s + torch.arange(s, device="cuda")).reshape(-1)
     slots = table.long().gather(1, pos.view(-1, s) // 16).view(-1) * 16 + pos % 16
     k2, v2 = kc.clone(), vc.clone()
-    announce("stream fused", s, h, kv)
+    announce("large batch fused", s, h, kv)
     q, _, _ = kernels.qk_norm_rope_store(qkv, qw, kw, cos[pos].contiguous(), sin[pos].contiguous(), 1e-6, k2, v2, slots,
                                          h, kv, D, need_kv=False)
     want = attention.paged_extend(q.view(len(lens), s, h, D), k2, v2, lens_t, table)
