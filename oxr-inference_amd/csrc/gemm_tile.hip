@@ -270,11 +270,11 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(1,
   }
 
   // Epilogue: lane (r, g) holds columns 4g .. 4g + 3 of a tile for token r.
+  if constexpr (EPI == kPartial) {
 #pragma unroll
-  for (int t = 0; t < kTM; ++t) {
-    const int tok = m0 + 16 * (wm * kTM + t) + r;
-    if (tok >= a.m) continue;
-    if constexpr (EPI == kPartial) {
+    for (int t = 0; t < kTM; ++t) {
+      const int tok = m0 + 16 * (wm * kTM + t) + r;
+      if (tok >= a.m) continue;
 #pragma unroll
       for (int j = 0; j < kTN; ++j) {
         const int64_t col = n0 + 16 * (wn * kTN + j) + 4 * g;
@@ -286,37 +286,62 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(1,
             if (col + e < a.n) dst[e] = acc[t][j][e];
         }
       }
-    } else {
-      constexpr int kOut = EPI == kSiluMul ? kTN / 2 : kTN;
+    }
+  } else {
+    constexpr int kOut = EPI == kSiluMul ? kTN / 2 : kTN;
+    float any = 0.f;  // NaN if any output is
+#pragma unroll
+    for (int t = 0; t < kTM; ++t) {
+      const int tok = m0 + 16 * (wm * kTM + t) + r;
+      if (tok >= a.m) continue;
 #pragma unroll
       for (int j = 0; j < kOut; ++j) {
         const int64_t col = n0 + 16 * (wn * kOut + j) + 4 * g;
-        // bf16 outputs in pairs (hardware rounding to nearest even).
-        uint32_t pair[2] = {pack_bf_hw(acc[t][j][0], acc[t][j][1]), pack_bf_hw(acc[t][j][2], acc[t][j][3])};
-        if constexpr (EPI == kSiluMul) {
-#pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            const f32x4 up = acc[t][kOut + j];
-            const uint32_t u = pack_bf_hw(up[2 * e], up[2 * e + 1]);
-            const uint32_t sl = pack_bf_hw(silu_bf16(lo_bf(pair[e])), silu_bf16(hi_bf(pair[e])));
-            pair[e] = pack_bf_hw(lo_bf(sl) * lo_bf(u), hi_bf(sl) * hi_bf(u));
-          }
-        }
         bf16_t* dst = a.y + (a.y_packed ? packed_offset(tok, col, a.n) : (int64_t)tok * a.ldy + col);
-        if (col + 3 < a.n) {
-          if constexpr (EPI == kAddResidual) {
-            const u32x2 old = *reinterpret_cast<const u32x2*>(dst);
-            pair[0] = pack_bf_hw(lo_bf(pair[0]) + lo_bf(old.x), hi_bf(pair[0]) + hi_bf(old.x));
-            pair[1] = pack_bf_hw(lo_bf(pair[1]) + lo_bf(old.y), hi_bf(pair[1]) + hi_bf(old.y));
+        const bool whole = col + 3 < a.n;
+        // bf16 outputs in pairs (hardware rounding to nearest even).
+        uint32_t pair[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          float lo = acc[t][j][2 * e], hi = acc[t][j][2 * e + 1];
+          if constexpr (EPI == kSiluMul) {
+            const f32x4 up = acc[t][kOut + j];
+            const uint32_t v = pack_bf_hw(lo, hi), u = pack_bf_hw(up[2 * e], up[2 * e + 1]);
+            const uint32_t sl = pack_bf_hw(silu_bf16(lo_bf(v)), silu_bf16(hi_bf(v)));
+            lo = lo_bf(sl) * lo_bf(u);
+            hi = hi_bf(sl) * hi_bf(u);
+          } else if constexpr (EPI == kAddResidual) {
+            const uint32_t v = pack_bf_hw(lo, hi);
+            uint32_t old = 0u;
+            if (whole) {
+              old = reinterpret_cast<const uint32_t*>(dst)[e];
+            } else {
+              for (int i = 0; i < 2; ++i)
+                if (col + 2 * e + i < a.n) old |= (uint32_t)dst[2 * e + i] << (16 * i);
+            }
+            lo = lo_bf(v) + lo_bf(old);
+            hi = hi_bf(v) + hi_bf(old);
           }
+          pair[e] = pack_bf_hw(lo, hi);
+          any = __builtin_elementwise_maximum(__builtin_elementwise_maximum(any, lo), hi);
+        }
+        if (whole) {
           *reinterpret_cast<u32x2*>(dst) = u32x2{pair[0], pair[1]};
         } else {
-          for (int e = 0; e < 4; ++e) {
-            if (col + e >= a.n) break;
-            uint32_t v = (pair[e >> 1] >> (16 * (e & 1))) & 0xffffu;
-            if constexpr (EPI == kAddResidual) v = pack_bf_hw(bf2f(v) + bf2f(dst[e]), 0.f) & 0xffffu;
-            dst[e] = (bf16_t)v;
-          }
+          for (int e = 0; e < 4; ++e)
+            if (col + e < a.n) dst[e] = (bf16_t)((pair[e >> 1] >> (16 * (e & 1))) & 0xffffu);
+        }
+      }
+    }
+    // The hardware's rounding keeps a NaN's payload; the 64-row kernel's NaN is canonical, so the lane's are made so.
+    if (any != any) {
+      for (int t = 0; t < kTM; ++t) {
+        const int tok = m0 + 16 * (wm * kTM + t) + r;
+        if (tok >= a.m) break;
+        for (int c = 0; c < 4 * kOut; ++c) {
+          const int64_t col = n0 + 16 * (wn * kOut + (c >> 2)) + 4 * g + (c & 3);
+          bf16_t* dst = a.y + (a.y_packed ? packed_offset(tok, col, a.n) : (int64_t)tok * a.ldy + col);
+          if (col < a.n && (*dst & 0x7fffu) > 0x7f80u) *dst = (bf16_t)0x7fc0u;
         }
       }
     }

@@ -54,11 +54,9 @@ def test_up_to_256_rows_equal_64_row_slices(m: int, k: int, n: int, epi: str) ->
 
 
 def test_silu_of_every_bf16_value() -> None:
-    """One-hot token rows and weights holding every finite bf16 gate value (up rows 1): the tiled kernel's
-    SiLU gives the bits of the 64-row kernel's expf and correctly rounded divide."""
-    bits = torch.arange(65_536, dtype=torch.int32)
-    values = (bits << 16).view(torch.float32)
-    values = values[torch.isfinite(values)].to(torch.bfloat16).cuda()
+    """One-hot token rows and weights holding every bf16 gate value, infinities and NaN among them (up rows 1): the
+    tiled kernel's SiLU gives the bits of the 64-row kernel's expf and correctly rounded divide."""
+    values = torch.arange(65_536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).cuda()
     w = torch.zeros(2 * values.numel(), 128, dtype=torch.bfloat16, device="cuda")
     w[:values.numel(), 0], w[values.numel():, 0] = values, 1.0
     x = torch.zeros(72, 128, dtype=torch.bfloat16, device="cuda")
@@ -68,6 +66,33 @@ def test_silu_of_every_bf16_value() -> None:
     torch.cuda.synchronize()
     assert torch.equal(got[:64].view(torch.int16), want.view(torch.int16))
     assert torch.equal(got[71].view(torch.int16), want[0].view(torch.int16))
+
+
+# Rows of NaN with payloads and signs of their own, of infinities and of their differences: the NaN outputs have the
+# canonical bits of the 64-row kernel, in whole column groups and in a last one of two columns.
+@pytest.mark.parametrize("m", [64, 72, 300])
+@pytest.mark.parametrize("n", [1024, 42])
+@pytest.mark.parametrize("epi", ["store", "silu", "add"])
+def test_nan_outputs_are_canonical(m: int, n: int, epi: str) -> None:
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    x, w, r = _rand(g, m, 256), _rand(g, 2 * n if epi == "silu" else n, 256, std=0.02), _rand(g, m, n)
+    odd = torch.tensor([0x7F81, -0x7F, 0x7FC1, -0x3B, 0x7F80, -0x80], dtype=torch.int16).view(torch.bfloat16).cuda()
+    w[:30:5, 3], w[33, 200], r[5, 30:36], r[m - 1, 9] = odd, float("inf"), odd, odd[1]
+    x[7, 11], x[m - 2, 17] = odd[3], float("inf")
+
+    def fn(x: torch.Tensor, r: torch.Tensor) -> torch.Tensor:
+        y = torch.empty(r.shape[0], n + 2, dtype=torch.bfloat16, device="cuda")[:, :n] if n == 42 else torch.empty_like(r)
+        if epi == "add":
+            return gemm.linear_add_(y.copy_(r), x, w)
+        return (gemm.linear if epi == "store" else gemm.linear_silu_mul)(x, w, out=y)
+
+    announce("nan", m, n, epi)
+    got, want = fn(x, r), torch.cat([fn(x[i:i + 64], r[i:i + 64]) for i in range(0, m, 64)])
+    torch.cuda.synchronize()
+    assert torch.equal(got.isnan(), want.isnan()) and bool(got.isnan().any())
+    assert bool((got.contiguous().view(torch.int16)[got.isnan()] == 0x7FC0).all())
+    if m <= 256:
+        assert torch.equal(got.contiguous().view(torch.int16), want.view(torch.int16))
 
 
 @pytest.mark.parametrize("m,k,n", [(257, 128, 40), (300, 2048, 4096), (513, 384, 1000), (1025, 1024, 12_288)])
