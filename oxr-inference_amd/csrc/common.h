@@ -103,6 +103,35 @@ __device__ __forceinline__ f32x4 mfma_16x16x32(const u32x4& a, const u32x4& b, c
                                                  0, 0);
 }
 
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ f32x16 mfma_32x32x16(const u32x4& a, const u32x4& b, const f32x16& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
+                                                 0, 0);
+}
+
+// One 1 KiB block from memory into LDS: lane i's 16 bytes at base + offset go to lds + 16 i (m0, the load's LDS
+// address, is read one wait state after it is written).  As inline asm the write is invisible to the compiler's
+// counters: left to the builtin, it cannot tell a ring's slots apart and waits for every block in flight before each
+// LDS read.  The caller orders the blocks with wait_vm and barriers instead.  Two things the compiler does not see
+// either: that m0 changes (the register is reserved, so a clobber only draws a warning), and that a vector
+// instruction may not write `base` in the 5 wait states before the load.  The build checks both in the generated code
+// (dma_faults in build.py): saving m0 and s_nop 4 in every block would cost the kernels that use it 2.5%.
+__device__ __forceinline__ void dma_block(const char* base, uint32_t offset, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base)
+               : "memory");
+}
+// The same, not kept in the caches.
+__device__ __forceinline__ void dma_block_nt(const char* base, uint32_t offset, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(offset), "s"(base)
+               : "memory");
+}
+
+// Until at most N of this wave's vector memory operations are outstanding (they complete in order).
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
 // 128-bit global loads/stores.  `nt` variants mark data that is streamed once
 // (weights, KV pages) so it does not evict reusable lines from L2.
 __device__ __forceinline__ u32x4 ld128(const void* p) { return *reinterpret_cast<const u32x4*>(p); }

@@ -27,7 +27,6 @@ namespace {
 
 enum Epilogue { kStore = 0, kSiluMul = 1, kAddResidual = 3, kPartial = 4 };
 
-
 struct KernelArgs {
   const bf16_t* x;
   const bf16_t* w;
@@ -37,20 +36,6 @@ struct KernelArgs {
   int m, tiles_m, tiles_n, k_slice, part_k;
   int x_packed, w_packed, y_packed;
 };
-
-// One 1 KiB block from memory into LDS (lane i's 16 bytes go to lds + 16 i).  As inline asm the write is
-// invisible to the compiler's counters: left to the builtin, it cannot tell the ring's slots apart and
-// waits for every block in flight before each LDS read.  The counted waits below order them instead.
-// (s_nop: the wait state between writing m0 and its use.)
-__device__ __forceinline__ void dma_block(const char* base, uint32_t offset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base)
-               : "memory");
-}
-
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 
 // silu(v) rounded to bf16, for v that is a bf16 value: the bits of bf16(v / (1 + expf(-v))) with a correctly
 // rounded divide for every such v (checked over all of them), in 9 instructions instead of about 45; in the

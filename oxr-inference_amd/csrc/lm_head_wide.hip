@@ -33,33 +33,12 @@
 namespace oxr {
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef short i16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kWaves = 8;
 constexpr int kGroup = 8;    // vocab tiles per group
 constexpr int kXSlots = 4;   // stages of token rows in LDS
 constexpr int kWBytes = kGroup * 2048;  // a stage of weight: 32 rows x 32 k per tile
-
-__device__ __forceinline__ f32x16 mfma_32x32x16(const u32x4& a, const u32x4& b, const f32x16& c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
-                                                 0, 0);
-}
-
-// One 1 KiB block from memory into LDS, invisible to the compiler's counters (see csrc/gemm_tile.hip).
-__device__ __forceinline__ void dma_block(const char* base, uint32_t offset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base)
-               : "memory");
-}
-__device__ __forceinline__ void dma_block_nt(const char* base, uint32_t offset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(offset), "s"(base)
-               : "memory");
-}
-
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 
 // Two packed bf16 values as signed 16-bit keys: ordered like the values, -0 equal to +0 (no NaN).
 __device__ __forceinline__ uint32_t key_pair(uint32_t p) {

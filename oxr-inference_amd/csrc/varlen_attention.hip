@@ -45,8 +45,6 @@
 namespace oxr {
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
 constexpr int kVD = 128;               // head dim
 constexpr int kVWaves = 4;             // waves per workgroup
 constexpr int kVRows = 32 * kVWaves;   // query rows per workgroup (all q heads of the kv head)
@@ -69,18 +67,6 @@ __device__ __forceinline__ uint32_t sched_take(uint32_t* p) {
   return __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-__device__ __forceinline__ f32x16 mfma_32x32x16(const u32x4& a, const u32x4& b, const f32x16& c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
-                                                 0, 0);
-}
-
-// One 1 KiB block from memory into LDS (lane i's 16 bytes to lds + 16 i), as inline asm: the compiler's
-// counters do not see it, so LDS reads are scheduled without waits for blocks in flight; the counted waits
-// and barriers of the tile loop order them.  (s_nop: wait states between the scalar writes and their use.)
-__device__ __forceinline__ void dma_block(const char* base, uint32_t offset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base)
-               : "memory");
-}
 __device__ __forceinline__ uint32_t lds_address(const bf16_t* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) bf16_t*)p;
 }
