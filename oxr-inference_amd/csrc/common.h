@@ -120,10 +120,18 @@ __device__ __forceinline__ void dma_block(const char* base, uint32_t offset, uin
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base)
                : "memory");
 }
-// The same, not kept in the caches.
-__device__ __forceinline__ void dma_block_nt(const char* base, uint32_t offset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(offset), "s"(base)
-               : "memory");
+// The same, not kept in the caches; kMask: with all lanes of the wave (`active` ~0) or none (0: nothing is loaded, but
+// the load is counted).  All are active before and after.
+template <bool kMask>
+__device__ __forceinline__ void dma_block_nt(const char* base, uint32_t offset, uint32_t lds, uint32_t active) {
+  if constexpr (kMask)
+    asm volatile("s_mov_b32 exec_lo, %3\n\ts_mov_b32 exec_hi, %3\n\ts_mov_b32 m0, %0\n\ts_nop 0\n\t"
+                 "global_load_lds_dwordx4 %1, %2 nt\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(offset), "s"(base),
+                 "s"(active)
+                 : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(offset), "s"(base)
+                 : "memory");
 }
 
 // Until at most N of this wave's vector memory operations are outstanding (they complete in order).

@@ -48,7 +48,11 @@ __device__ __forceinline__ uint32_t key_pair(uint32_t p) {
 }
 
 // TT: 32-token tiles (2, 4 or 8; rows past M are padding whose results nobody reads).
-template <int TT>
+// kMask: weight blocks past the range's end are not read.  Where the loads bound the kernel they cost what the others
+// do: 32,000 vocab rows are 4 tiles a CU, half a group (128 token rows 44.2 us, so 39.6; 151,936 rows 64 token rows
+// ids only 109.9 / 107.1).  At 256 token rows it makes no difference, and where a CU has one tile the mask is the
+// longer way to its next load (1000 vocab rows 31.0 / 32.3).
+template <int TT, bool kMask>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void lm_head_wide_kernel(
     const bf16_t* __restrict__ xp, int M, const bf16_t* __restrict__ w, int K, int64_t N,
     bf16_t* __restrict__ logits, int wide_stores, uint64_t* __restrict__ best_out) {
@@ -69,19 +73,21 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
   const int steps = K / 32;  // stages of a group
 
   // Loads.  Waves 0-3: blocks 4 wave .. + 3 of a weight stage (tile b / 2, 16-row half b % 2); waves 4-7:
-  // blocks of a token-row stage (16-row piece b).  Tiles past the range re-read its last one, stages past
-  // the last group repeat it: every stage issues the same number of loads.
+  // blocks of a token-row stage (16-row piece b).  Every stage issues the same number of loads: stages past the last
+  // group repeat it, tiles past the range's end are loaded with no lane active (kMask) or re-read its last one.
   const bool weight_wave = wave < 4;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
   const char* src[4];
+  uint32_t lanes[2] = {~0u, ~0u};  // of the loads of each of the wave's tiles: all or none
   int load_step = 0, load_group = 0, load_slot = 0;
   auto sources = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       if (weight_wave) {
         const int b = kWL * wave + u;
-        const int64_t vt = min(lo + (int64_t)min(load_group, groups - 1) * kGroup + (b >> 1), hi - 1);
-        src[u] = (const char*)(w + min(2 * vt + (b & 1), w_last) * (K * 16));
+        const int64_t vt = lo + (int64_t)min(load_group, groups - 1) * kGroup + (b >> 1);
+        src[u] = (const char*)(w + min(2 * min(vt, hi - 1) + (b & 1), w_last) * (K * 16));
+        lanes[u >> 1] = __builtin_amdgcn_readfirstlane(vt < hi ? ~0u : 0u);
       } else {
         const int b = kXL * (wave - 4) + u % kXL;
         src[u] = (const char*)(xp + (int64_t)min(b, (M + 15) / 16 - 1) * (K * 16));
@@ -93,7 +99,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
   const uint32_t my_ring = lds0 + (weight_wave ? kXSlots * kXBytes + kWL * wave * 1024 : kXL * (wave - 4) * 1024);
   auto issue1 = [&](int u) __attribute__((always_inline)) {
     const uint32_t at = my_ring + load_slot * my_bytes + u * 1024;
-    if (TT < 8 && weight_wave) dma_block_nt(src[u], lane_off, at);
+    if (TT < 8 && weight_wave) dma_block_nt<kMask>(src[u], lane_off, at, lanes[u >> 1]);
     else if (u < kXL || weight_wave) dma_block(src[u], lane_off, at);
   };
   auto issued = [&]() __attribute__((always_inline)) {
@@ -299,16 +305,17 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
   }
 }
 
-template <int TT>
+template <int TT, bool kMask>
 int launch(const bf16_t* xp, int M, const bf16_t* w, int64_t K, int64_t N, bf16_t* logits, uint64_t* best, int grid,
            hipStream_t s) {
   constexpr int lds = kXSlots * TT * 2048 + (TT == 8 ? 6 : 8) * kWBytes;
-  static const hipError_t attr = hipFuncSetAttribute((const void*)lm_head_wide_kernel<TT>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  const auto kernel = lm_head_wide_kernel<TT, kMask>;
+  static const hipError_t attr =
+      hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (attr != hipSuccess) return (int)attr;
   const int wide_stores = logits != nullptr && (uintptr_t)logits % 16 == 0 && N % 8 == 0;
-  hipLaunchKernelGGL(lm_head_wide_kernel<TT>, dim3((unsigned)grid), dim3(64 * kWaves), lds, s, xp, M, w, (int)K, N,
-                     logits, wide_stores, best);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * kWaves), lds, s, xp, M, w, (int)K, N, logits, wide_stores,
+                     best);
   return OXR_LAUNCH_STATUS();
 }
 
@@ -316,9 +323,10 @@ int launch(const bf16_t* xp, int M, const bf16_t* w, int64_t K, int64_t N, bf16_
 
 int launch_lm_head_wide(const bf16_t* xp, int M, const bf16_t* w, int64_t K, int64_t N, bf16_t* logits,
                         uint64_t* best, int grid, hipStream_t s) {
-  if (M <= 64) return launch<2>(xp, M, w, K, N, logits, best, grid, s);
-  if (M <= 128) return launch<4>(xp, M, w, K, N, logits, best, grid, s);
-  return launch<8>(xp, M, w, K, N, logits, best, grid, s);
+  const bool mask = (N + 31) / 32 > grid;
+  if (M <= 64) return (mask ? launch<2, true> : launch<2, false>)(xp, M, w, K, N, logits, best, grid, s);
+  if (M <= 128) return (mask ? launch<4, true> : launch<4, false>)(xp, M, w, K, N, logits, best, grid, s);
+  return launch<8, false>(xp, M, w, K, N, logits, best, grid, s);
 }
 
 }  // namespace oxr
