@@ -50,6 +50,7 @@ constexpr int kVWaves = 4;             // waves per workgroup
 constexpr int kVRows = 32 * kVWaves;   // query rows per workgroup (all q heads of the kv head)
 constexpr int kKeyTile = 64;           // keys per LDS stage
 constexpr int kLoadsPerWave = kKeyTile * kVD * 2 / 1024 / kVWaves;  // 1 KiB direct-to-LDS loads per wave and tensor
+constexpr int kNarrowHeads = 1 << 18;   // kv heads up to which the 63 rows behind a tile's first are within 4 GiB
 constexpr int kPersistentSlots = 64;   // persistent causal launch: workgroups per XCD (two per CU)
 
 // Work counters of the persistent causal launch, per launch slot (the host cycles through
@@ -100,6 +101,7 @@ __device__ __forceinline__ float row_max32(const f32x16 (&sv)[2]) {
 // no LDS after it, so the next item may start right away).  Thread 0 takes the next item number from
 // the counter `ctr` into `next` when the item's last two key tiles begin (or at once if it has no
 // work), late enough that the items are started in list order.
+template <bool kWide>
 __device__ __forceinline__ void varlen_item(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                                             const bf16_t* __restrict__ v, const int32_t* __restrict__ cu_seqlens,
                                             int H, int KV, float scale_log2, bf16_t* __restrict__ out, int pair,
@@ -150,7 +152,9 @@ __device__ __forceinline__ void varlen_item(const bf16_t* __restrict__ q, const 
   const int64_t row_bytes = (int64_t)KV * kVD * 2;
   const char* const kbase = (const char*)(k + ((int64_t)start * KV + kvh) * kVD);
   const char* const vbase = (const char*)(v + ((int64_t)start * KV + kvh) * kVD);
-  // Lane offsets of a whole tile: block u of the wave is 4 rows further (a scalar), its K rotation 4 chunks.
+  // Lane offsets of a whole tile: block u of the wave is 4 rows further (a scalar), its K rotation 4 chunks.  They hold
+  // 32 bits up to kNarrowHeads kv heads; beyond (kWide) a block's first row is added to the address instead.  (In one
+  // kernel for both, the longer code alone makes short sequences 3% slower: 3 prompts of 64 tokens 12.8 / 13.1 us.)
   const int row0 = 4 * kLoadsPerWave * wave + (lane >> 4), pos = lane & 15;
   const uint32_t row_off = (uint32_t)row0 * (uint32_t)row_bytes;
   uint32_t k_off[kLoadsPerWave];
@@ -161,6 +165,16 @@ __device__ __forceinline__ void varlen_item(const bf16_t* __restrict__ q, const 
     const char* const tile = (is_k ? kbase : vbase) + t * kKeyTile * row_bytes;
     const uint32_t at = lds_address(dst) + 1024 * kLoadsPerWave * wave;
     const int last = len - 1 - t * kKeyTile;  // the sequence's last key, in the tile
+    if constexpr (kWide) {
+      for (int u = 0; u < kLoadsPerWave; ++u) {
+        const int first = 4 * (kLoadsPerWave * wave + u), row = first + (lane >> 4);  // (`first` is wave-uniform)
+        dma_block(tile + min(first, last) * row_bytes,
+                  (uint32_t)min(row - first, max(last - first, 0)) * (uint32_t)row_bytes +
+                      16 * ((pos - (is_k ? row : 4 * row)) & 15),
+                  at + 1024 * u);
+      }
+      return;
+    }
     if (last >= kKeyTile - 1) {
 #pragma unroll
       for (int u = 0; u < kLoadsPerWave; ++u)
@@ -338,6 +352,7 @@ __device__ __forceinline__ void varlen_item(const bf16_t* __restrict__ q, const 
 // of the other groups' lists, in turn.  That balances the XCDs (measured: alone on their own lists,
 // their mean end times spread from 646 to 694 us in a 705 us launch) and mixed sequence lengths, whose
 // long sequences' pairs sit in few groups.
+template <bool kWide>
 __global__ __launch_bounds__(64 * kVWaves, 2) void varlen_attention_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
     const int32_t* __restrict__ cu_seqlens, int H, int KV, int num_qtiles, int num_pairs, int ring,
@@ -379,7 +394,7 @@ __global__ __launch_bounds__(64 * kVWaves, 2) void varlen_attention_kernel(
     }
     int next = 0;
     const int g = i / (2 * num_qtiles), gp = min(2, cnt - 2 * g), j = i - g * 2 * num_qtiles;
-    varlen_item(q, k, v, cu_seqlens, H, KV, scale_log2, out, lo + 2 * g + j % gp,
+    varlen_item<kWide>(q, k, v, cu_seqlens, H, KV, scale_log2, out, lo + 2 * g + j % gp,
                          num_qtiles - 1 - j / gp, s_k0, s_k1, s_v0, s_v1, base + grp * kSchedStride, &next);
     ++r;
     if (threadIdx.x == 0) s_item[r & 1] = next;
@@ -406,7 +421,7 @@ constexpr int kPWaves = 8;
 constexpr int kPRows = 32 * kPWaves;  // query rows per workgroup
 constexpr int kPLoadsPerWave = kKeyTile * kVD * 2 / 1024 / kPWaves;
 
-template <bool kCausal>
+template <bool kCausal, bool kWide>
 __global__ __launch_bounds__(64 * kPWaves, 1) void varlen_attention_pp_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
     const int32_t* __restrict__ cu_seqlens, int H, int KV, int num_qtiles, int num_pairs, int log2_parts,
@@ -461,6 +476,16 @@ __global__ __launch_bounds__(64 * kPWaves, 1) void varlen_attention_pp_kernel(
     const char* const tile = (is_k ? kbase : vbase) + t * kKeyTile * row_bytes;
     const uint32_t at = lds_address(dst) + 1024 * kPLoadsPerWave * wave;
     const int last = len - 1 - t * kKeyTile;  // the sequence's last key, in the tile
+    if constexpr (kWide) {
+      for (int u = 0; u < kPLoadsPerWave; ++u) {
+        const int first = 4 * (kPLoadsPerWave * wave + u), row = first + (lane >> 4);  // (`first` is wave-uniform)
+        dma_block(tile + min(first, last) * row_bytes,
+                  (uint32_t)min(row - first, max(last - first, 0)) * (uint32_t)row_bytes +
+                      16 * ((pos - (is_k ? row : 4 * row)) & 15),
+                  at + 1024 * u);
+      }
+      return;
+    }
     if (last >= kKeyTile - 1) {
 #pragma unroll
       for (int u = 0; u < kPLoadsPerWave; ++u)
@@ -675,6 +700,8 @@ extern "C" int oxr_varlen_attention(const oxr_bf16* q, const oxr_bf16* k, const 
   OXR_RETURN_IF(head_dim != kVD || num_heads % num_kv_heads != 0, OXR_ERR_UNSUPPORTED);
   const int G = num_heads / num_kv_heads;
   OXR_RETURN_IF(8 % G != 0, OXR_ERR_UNSUPPORTED);  // G in {1, 2, 4, 8}
+  OXR_RETURN_IF(num_kv_heads > 1 << 22, OXR_ERR_UNSUPPORTED);  // a block's 4 rows lie within 4 GiB
+  const bool wide = num_kv_heads > kNarrowHeads;
   if (num_seqs == 0 || max_len == 0) return OXR_OK;
   OXR_RETURN_IF(!q || !k || !v || !cu_seqlens || !out, OXR_ERR_INVALID_ARG);
   OXR_RETURN_IF(((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) % 16 != 0 || (uintptr_t)out % 8 != 0,
@@ -693,14 +720,16 @@ extern "C" int oxr_varlen_attention(const oxr_bf16* q, const oxr_bf16* k, const 
   if (!causal) {
     const int parts = log2_parts(num_kv_heads, num_pairs, num_qtiles);
     const dim3 grid((unsigned)query_tile_blocks(num_pairs, num_qtiles, parts));
-    hipLaunchKernelGGL(varlen_attention_pp_kernel<false>, grid, dim3(64 * kPWaves), 0, s, q, k, v, cu_seqlens,
+    const auto kernel = wide ? varlen_attention_pp_kernel<false, true> : varlen_attention_pp_kernel<false, false>;
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * kPWaves), 0, s, q, k, v, cu_seqlens,
                        num_heads, num_kv_heads, num_qtiles, num_pairs, parts, scale_log2, out);
   } else {
     // Two workgroups per CU, or fewer when the largest XCD group has fewer items.
     static std::atomic<uint32_t> launches{0};
     const int ring = (int)(launches.fetch_add(1u, std::memory_order_relaxed) % kSchedRing);
     const int per_xcd = (int)std::min<int64_t>(kPersistentSlots, (int64_t)((num_pairs + 7) / 8) * num_qtiles);
-    hipLaunchKernelGGL(varlen_attention_kernel, dim3(8 * per_xcd), dim3(64 * kVWaves), 0, s, q, k, v, cu_seqlens,
+    const auto kernel = wide ? varlen_attention_kernel<true> : varlen_attention_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3(8 * per_xcd), dim3(64 * kVWaves), 0, s, q, k, v, cu_seqlens,
                        num_heads, num_kv_heads, num_qtiles, num_pairs, ring, scale_log2, out);
   }
   return OXR_LAUNCH_STATUS();

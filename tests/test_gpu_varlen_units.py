@@ -36,3 +36,24 @@ def test_bidirectional_a_million_one_token_sequences() -> None:
     out = attention.varlen(q, k, v, torch.arange(n + 1, dtype=torch.int32, device="cuda"), 1, causal=False)
     torch.cuda.synchronize()
     assert torch.equal(out, v)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+def test_rows_past_32_bit_offsets(causal: bool) -> None:
+    """270,000 kv heads: 63 rows of a key tile are more than 2^32 bytes.  A few heads against float64, with a tile cut by
+    the sequence's end; tolerance: bf16 rounding of the output and of the probabilities (2^-8 of each)."""
+    n, kv = 65, 270_000
+    g = torch.Generator(device="cuda").manual_seed(61)
+    q, k, v = (torch.empty(n, kv, 128, dtype=torch.bfloat16, device="cuda").normal_(generator=g) for _ in range(3))
+    announce("varlen wide rows", n, kv, causal)
+    out = attention.varlen(q, k, v, torch.tensor([0, n], dtype=torch.int32, device="cuda"), n, causal=causal)
+    torch.cuda.synchronize()
+    for head in (0, 1, 135_000, kv - 1):
+        qd, kd, vd = (t[:, head].double() for t in (q, k, v))
+        scores = qd @ kd.t() * 128 ** -0.5
+        if causal:
+            scores.masked_fill_(torch.ones(n, n, dtype=torch.bool, device="cuda").triu(1), float("-inf"))
+        p = torch.softmax(scores, -1)
+        want = p @ vd
+        err = (out[:, head].double() - want).abs()
+        assert bool((err <= 2.0 ** -8 * (want.abs() + p @ vd.abs()) + 1e-5).all()), head
