@@ -29,11 +29,12 @@ __global__ __launch_bounds__(kMaxHeads* kLanesPerHead) void qk_norm_rope_store_k
     const bf16_t* __restrict__ qkv, const bf16_t* __restrict__ q_weight, const bf16_t* __restrict__ k_weight,
     const bf16_t* __restrict__ cos_table, const bf16_t* __restrict__ sin_table, float eps,
     bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache, const int64_t* __restrict__ slots,
-    int64_t num_slots, int num_heads, int num_kv_heads, bf16_t* __restrict__ q_out, bf16_t* __restrict__ k_out,
-    bf16_t* __restrict__ v_out, const int64_t* __restrict__ positions, int64_t table_rows) {
+    int64_t num_slots, int num_heads, int num_kv_heads, int first_head, bf16_t* __restrict__ q_out,
+    bf16_t* __restrict__ k_out, bf16_t* __restrict__ v_out, const int64_t* __restrict__ positions,
+    int64_t table_rows) {
   const int heads_per_token = num_heads + 2 * num_kv_heads;
   const int64_t t = blockIdx.x;
-  const int first = (int)(blockIdx.y * blockDim.x + threadIdx.x) / kLanesPerHead;
+  const int first = first_head + (int)(blockIdx.y * blockDim.x + threadIdx.x) / kLanesPerHead;
   const int s = threadIdx.x % kLanesPerHead;
   // Lanes past the token's last head keep running on that head so every lane
   // takes part in the exchanges below; they store nothing.
@@ -87,18 +88,21 @@ int launch_qk(const oxr_bf16* qkv, const oxr_bf16* q_weight, const oxr_bf16* k_w
                 OXR_ERR_INVALID_ARG);
   const int64_t heads = num_heads + 2 * (int64_t)num_kv_heads;
   const int64_t chunks = (heads + kMaxHeads - 1) / kMaxHeads;
-  OXR_RETURN_IF(chunks > 65535, OXR_ERR_UNSUPPORTED);
+  OXR_RETURN_IF(heads > INT32_MAX - kMaxHeads, OXR_ERR_UNSUPPORTED);
   const dim3 block(kWave * (unsigned)((std::min<int64_t>(heads, kMaxHeads) + 3) / 4));
   hipStream_t s = (hipStream_t)stream;
   const auto kernel = k_out ? qk_norm_rope_store_kernel<true> : qk_norm_rope_store_kernel<false>;
   constexpr int64_t kSlice = 1 << 23;  // tokens per launch: a launch holds less than 2^32 threads in x
+  constexpr int64_t kChunks = 65535;   // and head chunks: its blocks in y
   for (int64_t t0 = 0; t0 < n; t0 += kSlice) {
-    const dim3 grid((unsigned)std::min(kSlice, n - t0), (unsigned)chunks);
     const int64_t table = positions ? 0 : t0 * (kHeadDim / 2), kv = t0 * num_kv_heads * kHeadDim;
-    hipLaunchKernelGGL(kernel, grid, block, 0, s, qkv + t0 * heads * kHeadDim, q_weight, k_weight, cos + table,
-                       sin + table, eps, k_cache, v_cache, slots + t0, num_slots, num_heads, num_kv_heads,
-                       q_out + t0 * num_heads * kHeadDim, k_out ? k_out + kv : nullptr, k_out ? v_out + kv : nullptr,
-                       positions ? positions + t0 : nullptr, table_rows);
+    for (int64_t c0 = 0; c0 < chunks; c0 += kChunks) {
+      const dim3 grid((unsigned)std::min(kSlice, n - t0), (unsigned)std::min(kChunks, chunks - c0));
+      hipLaunchKernelGGL(kernel, grid, block, 0, s, qkv + t0 * heads * kHeadDim, q_weight, k_weight, cos + table,
+                         sin + table, eps, k_cache, v_cache, slots + t0, num_slots, num_heads, num_kv_heads,
+                         (int)(c0 * kMaxHeads), q_out + t0 * num_heads * kHeadDim, k_out ? k_out + kv : nullptr,
+                         k_out ? v_out + kv : nullptr, positions ? positions + t0 : nullptr, table_rows);
+    }
   }
   return OXR_LAUNCH_STATUS();
 }

@@ -168,3 +168,27 @@ def test_non_finite_rows_bit_exact() -> None:
                                                   np.zeros((n, 1, KV, D), np.uint16), np.zeros((n, 1, KV, D), np.uint16),
                                                   slots, H, KV, D, need_kv=True)
     assert np.array_equal(_bits(q), wq) and np.array_equal(_bits(k), wk) and np.array_equal(_bits(v), wv)
+
+
+def test_more_heads_than_a_launch_has_rows_of_blocks() -> None:
+    """Over 65,535 x 16 heads a token: the last of them equal, bit for bit, a call that holds only those."""
+    n, h, tail, d = 2, 65_535 * 16 + 30, 40, 128
+    g = torch.Generator(device="cuda").manual_seed(27)
+    qkv = torch.empty(n, h + 2, d, dtype=torch.bfloat16, device="cuda").normal_(generator=g)
+    qw, kw = (torch.rand(d, generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    angles = torch.rand(n, d // 2, generator=g, device="cuda")
+    cos, sin = angles.cos().to(torch.bfloat16), angles.sin().to(torch.bfloat16)
+    slots = torch.tensor([5, 2], device="cuda")
+    announce("wide tokens", n, h)
+
+    def run(x: torch.Tensor, heads: int):
+        kc, vc = (torch.zeros(1, 16, 1, d, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        q, k, v = kernels.qk_norm_rope_store(x.reshape(n, -1), qw, kw, cos, sin, 1e-6, kc, vc, slots, heads, 1, d,
+                                             need_kv=True)
+        torch.cuda.synchronize()
+        return q.view(n, heads, d), k, v, kc, vc
+
+    got, want = run(qkv, h), run(qkv[:, h - tail:].contiguous(), tail)
+    assert torch.equal(got[0][:, h - tail:].reshape(-1).view(torch.int16), want[0].reshape(-1).view(torch.int16))
+    for a, b in zip(got[1:], want[1:]):
+        assert torch.equal(a.reshape(-1).view(torch.int16), b.reshape(-1).view(torch.int16))
