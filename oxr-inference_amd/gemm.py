@@ -111,10 +111,10 @@ def _check(x: Rows, w: Weight, name: str) -> torch.device:
 
 def _run(x: Rows, w: Weight, n: int, epilogue: int, y: Rows, device: torch.device) -> None:
     m = x.shape[0]
-    if m == 0:
-        return
     packed = isinstance(w, PackedMatrix)
     _lib.require(packed or not isinstance(y, PackedMatrix), "packed output needs a packed w")
+    if m == 0:
+        return
     flags = (X_PACKED if isinstance(x, PackedMatrix) else 0) | (Y_PACKED if isinstance(y, PackedMatrix) else 0)
     _lib.require(not flags or m <= MAX_ROWS, f"packed rows: at most {MAX_ROWS} per call")
     ldx = 0 if isinstance(x, PackedMatrix) else x.stride(0)
