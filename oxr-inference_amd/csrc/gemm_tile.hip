@@ -263,13 +263,8 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(1,
 #pragma unroll
       for (int j = 0; j < kTN; ++j) {
         const int64_t col = n0 + 16 * (wn * kTN + j) + 4 * g;
-        float* dst = a.part + ((int64_t)split * a.m + tok) * a.n + col;
-        if (col + 3 < a.n) {
-          *reinterpret_cast<f32x4*>(dst) = acc[t][j];
-        } else {
-          for (int e = 0; e < 4; ++e)
-            if (col + e < a.n) dst[e] = acc[t][j][e];
-        }
+        if (col < a.n)  // n is a multiple of 4
+          *reinterpret_cast<f32x4*>(a.part + ((int64_t)split * a.m + tok) * a.n + col) = acc[t][j];
       }
     }
   } else {
@@ -351,9 +346,11 @@ int launch(const TileArgs& t, int parts, hipStream_t s) {
 
 template <int EPI>
 int dispatch(const TileArgs& t, int tile, int parts, hipStream_t s) {
+  if constexpr (EPI != kPartial) {  // partial sums are never one chain
+    if (tile == 0) return launch<256, 256, 2, 4, 2, 64, false, EPI>(t, parts, s);
+    if (tile == 1) return launch<256, 128, 4, 2, 3, 64, false, EPI>(t, parts, s);
+  }
   switch (tile) {
-    case 0: return launch<256, 256, 2, 4, 2, 64, false, EPI>(t, parts, s);
-    case 1: return launch<256, 128, 4, 2, 3, 64, false, EPI>(t, parts, s);
     case 2: return launch<128, 128, 4, 2, 4, 64, true, EPI>(t, parts, s);
     case 3: return launch<128, 64, 4, 2, 3, 128, true, EPI>(t, parts, s);
     case 4: return launch<64, 64, 4, 2, 4, 128, true, EPI>(t, parts, s);
