@@ -9,6 +9,7 @@
 #include <stdint.h>
 
 #include "../../include/oxr_verify.h"
+#include "per_device.h"
 
 namespace oxr {
 
@@ -166,3 +167,16 @@ __device__ __forceinline__ int64_t packed_offset(int64_t row, int64_t k, int64_t
   } while (0)
 
 #define OXR_LAUNCH_STATUS() ((int)hipGetLastError())
+
+namespace oxr {
+// Lets `kernel` be launched with `bytes` of dynamic LDS on the current device (an attribute of the kernel there);
+// `done` belongs to the kernel.  Returns 0 or an error status.
+inline int allow_dynamic_lds(std::atomic<uint64_t>& done, const void* kernel, int bytes) {
+  int device = 0;
+  const hipError_t e = hipGetDevice(&device);
+  if (e != hipSuccess) return (int)e;
+  return once_per_device(done, device, [&] {
+    return (int)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  });
+}
+}  // namespace oxr

@@ -545,13 +545,9 @@ template <int NB, int K, bool PW>
 int launch_lm_head_lds(const bf16_t* x, int64_t ldx, int M, const bf16_t* w, int64_t N, bf16_t* logits,
                        uint64_t* best, int grid, hipStream_t s) {
   constexpr size_t lds = (size_t)NB * 16 * K * sizeof(bf16_t);
-  static bool attr_set = false;  // per instantiation; setting it twice is harmless
-  if (!attr_set) {
-    const hipError_t e = hipFuncSetAttribute((const void*)lm_head_lds_kernel<NB, K, PW>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return (int)e;
-    attr_set = true;
-  }
+  static std::atomic<uint64_t> lds_allowed{0};
+  const int st = allow_dynamic_lds(lds_allowed, (const void*)lm_head_lds_kernel<NB, K, PW>, (int)lds);
+  if (st) return st;
   hipLaunchKernelGGL((lm_head_lds_kernel<NB, K, PW>), dim3((unsigned)grid), dim3(64 * kLmWaves), lds, s, x, ldx, M, w,
                      N, logits, N, best);
   return OXR_LAUNCH_STATUS();

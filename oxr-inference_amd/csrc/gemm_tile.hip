@@ -332,9 +332,9 @@ template <int BM, int BN, int WM, int WN, int STAGES, int KC, bool kParts, int E
 int launch(const TileArgs& t, int parts, hipStream_t s) {
   constexpr size_t lds = (size_t)STAGES * (BM + BN) * 2 * KC;
   const auto kernel = gemm_tile_kernel<BM, BN, WM, WN, STAGES, KC, kParts, EPI>;
-  static const hipError_t attr =
-      hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (attr != hipSuccess) return (int)attr;
+  static std::atomic<uint64_t> lds_allowed{0};
+  const int st = allow_dynamic_lds(lds_allowed, (const void*)kernel, (int)lds);
+  if (st) return st;
   constexpr int kCols = EPI == kSiluMul ? BN / 2 : BN;
   const int64_t tiles_m = (t.m + BM - 1) / BM, tiles_n = (t.n + kCols - 1) / kCols;
   const int k_slice = (int)(t.k / t.k_splits);

@@ -310,9 +310,9 @@ int launch(const bf16_t* xp, int M, const bf16_t* w, int64_t K, int64_t N, bf16_
            hipStream_t s) {
   constexpr int lds = kXSlots * TT * 2048 + (TT == 8 ? 6 : 8) * kWBytes;
   const auto kernel = lm_head_wide_kernel<TT, kMask>;
-  static const hipError_t attr =
-      hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  if (attr != hipSuccess) return (int)attr;
+  static std::atomic<uint64_t> lds_allowed{0};
+  const int st = allow_dynamic_lds(lds_allowed, (const void*)kernel, lds);
+  if (st) return st;
   const int wide_stores = logits != nullptr && (uintptr_t)logits % 16 == 0 && N % 8 == 0;
   hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * kWaves), lds, s, xp, M, w, (int)K, N, logits, wide_stores,
                      best);
