@@ -371,8 +371,7 @@ int oxr_qk_norm_rope_paged_extend_static(const oxr_bf16* qkv, const oxr_bf16* q_
  *   OXR_EPI_ADD_RESIDUAL y = bf16(bf16(x @ w^T) + y), in place: the residual
  *                        add of _add_rms_norm (language.py:94-99)
  * x bf16 [m, ldx] (first k columns used), w bf16 [rows, k] row-major, fp32
- * accumulation.  m <= 256, k a
- * multiple of 128, x and w 16-byte aligned.
+ * accumulation.  m <= 256, k a multiple of 128, x and w 16-byte aligned.
  */
 #define OXR_EPI_STORE 0
 #define OXR_EPI_SILU_MUL 1
@@ -382,8 +381,11 @@ int oxr_gemm_bf16(const oxr_bf16* x, int64_t ldx, int64_t m, const oxr_bf16* w, 
 
 /*
  * (4a'') The same for any number of token rows (a prompt's projections), the
- * weight row-major or (w_packed != 0) packed.  Above 256 rows each output is
- * one chain of fp32 products over k.
+ * weight row-major or (w_packed != 0) packed.  Up to 256 rows the results are
+ * those of (4a), whose order of sums does not depend on the number of rows.
+ * Above, each output is one chain of fp32 products over k, so a row's last
+ * bits may differ from those of a call of at most 256 rows; with k or ldx over
+ * 2^22, which the tiled kernel does not take, the order of (4a) stays.
  */
 int oxr_gemm_bf16_tall(const oxr_bf16* x, int64_t ldx, int64_t m, const oxr_bf16* w, int64_t k, int64_t n,
                        int32_t epilogue, oxr_bf16* y, int64_t ldy, int32_t w_packed, oxr_stream_t stream);

@@ -14,10 +14,10 @@
 // * Within a stage fragments are read two products ahead, with a scheduling barrier per step: left alone
 //   the compiler reads each fragment right before its use and waits for the LDS latency 16 times a stage
 //   (256 x 256 tile, K = 2048, 4096 x 4096: 65 us; read ahead 56).
-// What bounds it.  Large tiles (4096 rows): the matrix cores are busy 62% of the CU cycles (256 x 256) and 58%
-// (256 x 128), LDS reads 23 to 29%; the rest is stage barriers and waits that two waves per SIMD do not cover.
+// What bounds it.  Large tiles (4096 rows): the matrix cores are busy 61 to 64% of the CU cycles (256 x 256) and 55%
+// (256 x 128), LDS reads 23 to 28%; the rest is stage barriers and waits that two waves per SIMD do not cover.
 // 4 waves of 128 x 128 read a quarter less LDS but leave one wave per SIMD: 71 us against 56.  Small tiles (up to
-// 256 rows): matrix cores 33%, LDS 24%; the chain of stages waits on memory (see kPer below).
+// 256 rows): matrix cores 28 to 38%, LDS 28%; the chain of stages waits on memory (see kPer below).
 #include <algorithm>
 
 #include "gemm_tile.h"

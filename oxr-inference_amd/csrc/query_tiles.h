@@ -11,7 +11,7 @@
 // from each round of 8 to the next, so over 8 pairs every XCD takes exactly num_qtiles tiles, and only the last,
 // incomplete 8 leave workgroups without one.  (An empty workgroup costs the dispatcher as much as a short one: with a
 // slot for every part whether or not it holds a tile, 2048 sequences of 30 tokens with 5 kv heads took 1992 us
-// against 260, and with parts that stay on their XCD 7 of 600 tokens with 6 took 49 against 31.)
+// against 252, and with parts that stay on their XCD 7 of 600 tokens with 6 took 49 against 31.)
 #pragma once
 
 #include <algorithm>

@@ -26,10 +26,10 @@
 //   exp2-domain online softmax, then O^T += V^T P^T (16 MFMAs: 4 dim blocks x
 //   4 key steps; P^T is used as computed: k slot 8h + 4p + j of key step ks
 //   stands for key 16ks + 8p + 4h + j).  The V^T fragments come from gfx950's
-//   transposing LDS read (ds_read_b64_tr_b16) of the row-major V tile.  The
-//   QK^T products of tile t + 1 are issued among tile t's exponentials (K is
-//   staged one tile ahead of V), so the matrix cores and the vector unit of a
-//   wave overlap.
+//   transposing LDS read (ds_read_b64_tr_b16) of the row-major V tile.  LDS
+//   fragments are read ahead of their products, and each key step's
+//   exponentials stand behind the products of the step before, so the matrix
+//   cores and the vector unit of a wave overlap.
 // * Causal: key tiles above a wave's last row are skipped, tiles that cross a
 //   row's diagonal are masked per element; keys past the sequence are masked.
 // Causal prefill runs this 4-wave kernel as a persistent launch whose

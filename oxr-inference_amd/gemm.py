@@ -90,7 +90,7 @@ def pack_weight(w: torch.Tensor) -> PackedMatrix:
 
 EPI_STORE, EPI_SILU_MUL, EPI_ADD_RESIDUAL = 0, 1, 3
 X_PACKED, Y_PACKED = 1, 2  # OXR_GEMM_X_PACKED, OXR_GEMM_Y_PACKED
-MAX_ROWS = 256  # token rows of a call with packed rows or k-split partials
+MAX_ROWS = 256  # token rows of a call with packed rows or k-split partials, or whose sums keep their order
 
 
 def _tensor(a: Weight) -> torch.Tensor:
@@ -136,7 +136,12 @@ def _check_out(out: Rows, m: int, n: int, name: str) -> None:
 
 
 def linear(x: Rows, w: Weight, out: Rows | None = None) -> Rows:
-    """``x @ w.T`` in bf16 with fp32 accumulation (``F.linear`` without bias)."""
+    """``x @ w.T`` in bf16 with fp32 accumulation (``F.linear`` without bias).
+
+    Up to ``MAX_ROWS`` rows the order of a row's sums does not depend on how many rows share its call.  Beyond, each
+    output is one chain of products over k, another order: the same row in a call of at most 256 rows and in a larger
+    one may differ in its last bits.  A program that needs equal bits whatever the size of its prompt chunks passes
+    at most ``MAX_ROWS`` rows at a time."""
     device = _check(x, w, "linear")
     n = w.shape[0]
     if out is None:
@@ -147,7 +152,8 @@ def linear(x: Rows, w: Weight, out: Rows | None = None) -> Rows:
 
 
 def linear_silu_mul(x: Rows, w: Weight, out: Rows | None = None) -> Rows:
-    """``silu(g) * u`` where ``[g | u] = x @ w.T`` (``w`` is the fused gate_up weight, gate rows first)."""
+    """``silu(g) * u`` where ``[g | u] = x @ w.T`` (``w`` is the fused gate_up weight, gate rows first).
+    The order of the sums changes above ``MAX_ROWS`` rows, as in :func:`linear`."""
     device = _check(x, w, "linear_silu_mul")
     _lib.require(w.shape[0] % 2 == 0, "linear_silu_mul: w must hold gate and up rows")
     n = w.shape[0] // 2
@@ -159,7 +165,8 @@ def linear_silu_mul(x: Rows, w: Weight, out: Rows | None = None) -> Rows:
 
 
 def linear_add_(residual: torch.Tensor, x: Rows, w: Weight) -> torch.Tensor:
-    """``residual = bf16(bf16(x @ w.T) + residual)``, in place; returns ``residual``."""
+    """``residual = bf16(bf16(x @ w.T) + residual)``, in place; returns ``residual``.  The order of the sums
+    changes above ``MAX_ROWS`` rows, as in :func:`linear`."""
     device = _check(x, w, "linear_add_")
     n = w.shape[0]
     _lib.require(residual.shape == (x.shape[0], n) and residual.dtype == torch.bfloat16 and residual.stride(1) == 1,
