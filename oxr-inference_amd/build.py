@@ -135,7 +135,10 @@ def dma_faults(asm: str) -> list[str]:
                 faults.append(f"load into LDS without its own write of m0: {text}")
                 continue
             blessed.add(i - 2)
-            if written_above(i - 1, _BASE_STATES, _sgprs(text.split(",", 1)[1])):
+            base = _sgprs(text.split(",", 1)[1])
+            if not base:
+                faults.append(f"load into LDS from a base in other than numbered registers: {text}")
+            elif written_above(i - 1, _BASE_STATES, base):
                 faults.append(f"vector write of the base address just before: {text}")
     faults += [f"m0 used elsewhere: {text}" for i, text in enumerate(lines)
                if re.search(r"\bm0\b", text) and i not in blessed]

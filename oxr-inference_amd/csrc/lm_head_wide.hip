@@ -17,10 +17,10 @@
 // * Epilogue per group: bf16 logits as 16-byte stores (two lanes' halves exchanged), and the running best of
 //   each token as one 32-bit integer (signed bf16 key, column) per lane: 4 instructions a logit.
 //
-// Kernel alone at vocab 151,936, hidden 2048, ids only, us: 256 rows 165 (185 with logits), 96 rows 119, 64 rows 104
-// (6.0 TB/s).  Up to 128 rows the HBM stream bounds it; the weight is loaded non-temporally there (64 rows: 111 without).  At
-// 256 rows the parts by themselves take 96 (products: the clock falls from 2.5 to 2.0 GHz under them), 45
-// (fragment reads) and 118 (loads); what is left is that a wave whose loads wait to be issued does not
+// Kernel alone at vocab 151,936, hidden 2048, ids only, us: 256 rows 165 (185 with logits), 96 rows 119, 64 rows
+// 104 (6.0 TB/s).  Up to 128 rows the HBM stream bounds it; the weight is loaded non-temporally there (64 rows: 111
+// without).  At 256 rows the parts by themselves take 96 (products: the clock falls from 2.5 to 2.0 GHz under
+// them), 45 (fragment reads) and 118 (loads); what is left is that a wave whose loads wait to be issued does not
 // multiply.  Neither the ring's depth, nor wave priorities, nor non-temporal weight loads (171) move it.
 //
 // Each logit is one chain of products over k in ascending order, whatever the number of rows.

@@ -40,3 +40,4 @@ def test_refuses_other_uses_of_m0() -> None:
     assert len(faults(LOAD.format("") + "\ts_mov_b32 m0, s3\n\tv_movrels_b32 v1, v2\n")) == 1
     assert len(faults(LOAD.format("") + "\ts_add_u32 s4, m0, 4\n")) == 1
     assert len(faults("\tglobal_load_lds_dwordx4 v1, s[10:11]\n")) == 1  # m0 as someone else left it
+    assert len(faults(LOAD.format("").replace("s[10:11]", "vcc"))) == 1  # a base the check does not follow
